@@ -23,10 +23,13 @@ struct PairMeta {
 };
 
 // A segment of one bra row: items t0 .. t0 + n - 1 of the list, all with
-// the bra pair of row `row`.
+// the bra pair of row `row`.  2^ls lanes of a wavefront share each item and
+// divide its ket primitive pairs (k_eri_seg, k_eri_gc, k_eri_gck; ls = 0 in
+// the lists of the other kernels).
 struct SegDesc {
     long long t0;
-    int row, n;
+    int row;
+    int n : 26, ls : 6;
 };
 
 struct EriArgs {
@@ -699,6 +702,85 @@ __global__ void __launch_bounds__(256) k_eri(EriArgs g) {
         eri_item<LA, LB, LC, LD, MODE>(g, t);
 }
 
+// Sums over the lanes that share one item.  The 2^ls lanes of an item are
+// those that differ in lane bits 5, 4, .. 6 - ls, so step S of a reduction
+// exchanges with the lane whose bit 5 - S differs, whatever ls is.
+// halve: two values x (kept by lanes with the bit clear) and y (kept by the
+// others); returns the kept one summed over the pair of lanes.  On the two
+// widest steps one v_permlane swap per 32-bit half moves both.
+// full: x summed over the pair, in both lanes.
+template <int S>
+__device__ __forceinline__ unsigned lane_xchg(unsigned v) {
+    if constexpr (S == 2) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xf, 0xf, true);        // row_ror:8 = lane ^ 8
+    else if constexpr (S == 3) return __builtin_amdgcn_ds_swizzle(v, (4 << 10) | 0x1f);     // lane ^ 4
+    else if constexpr (S == 4) return __builtin_amdgcn_mov_dpp(v, 0x4e, 0xf, 0xf, true);    // quad_perm [2,3,0,1]
+    else return __builtin_amdgcn_mov_dpp(v, 0xb1, 0xf, 0xf, true);                          // quad_perm [1,0,3,2]
+}
+template <int S>
+__device__ __forceinline__ double lane_halve(double x, double y, int lane) {
+    const unsigned long long a = __builtin_bit_cast(unsigned long long, x);
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, y);
+    if constexpr (S < 2) {
+        const auto swap = [](unsigned p, unsigned q) {
+            if constexpr (S == 0) return __builtin_amdgcn_permlane32_swap(p, q, false, false);
+            else return __builtin_amdgcn_permlane16_swap(p, q, false, false);
+        };
+        const auto lo = swap((unsigned)a, (unsigned)b), hi = swap((unsigned)(a >> 32), (unsigned)(b >> 32));
+        return __builtin_bit_cast(double, (unsigned long long)hi[0] << 32 | lo[0]) +
+               __builtin_bit_cast(double, (unsigned long long)hi[1] << 32 | lo[1]);
+    } else {
+        const bool up = lane >> (5 - S) & 1;
+        const unsigned long long send = up ? a : b;
+        const unsigned lo = lane_xchg<S>((unsigned)send), hi = lane_xchg<S>((unsigned)(send >> 32));
+        return (up ? y : x) + __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+    }
+}
+template <int S>
+__device__ __forceinline__ double lane_full(double x, int lane) {
+    return lane_halve<S>(x, x, lane);
+}
+
+// acc holds N values for each of M2 x M1 members (member (i, j) at
+// (i M1 + j) N).  Sums over the item's lanes, the first steps halving the
+// j range a lane keeps, the next the i range, the last plain sums: afterwards
+// the lane holds members i0 .. i0 + ni - 1, j0 .. j0 + nj - 1 at indices
+// from (0, 0); of the lanes left with equal members one has first = true.
+template <int M2, int M1, int N, int S = 0>
+__device__ __forceinline__ void lane_reduce(double* acc, int ls, int lane, int& i0, int& ni, int& j0, int& nj,
+                                            bool& first) {
+    constexpr int LJ = M1 == 4 ? 2 : M1 == 2 ? 1 : 0, LI = M2 == 4 ? 2 : M2 == 2 ? 1 : 0;
+    static_assert(M1 == 1 << LJ && M2 == 1 << LI, "member counts are 1, 2 or 4");
+    if (S >= ls) return;
+    const int up = lane >> (5 - S) & 1;
+    if constexpr (S < LJ) {
+        constexpr int h = M1 >> (S + 1);
+#pragma unroll
+        for (int i = 0; i < M2; ++i)
+#pragma unroll
+            for (int j = 0; j < h; ++j)
+#pragma unroll
+                for (int e = 0; e < N; ++e)
+                    acc[(i * M1 + j) * N + e] =
+                        lane_halve<S>(acc[(i * M1 + j) * N + e], acc[(i * M1 + j + h) * N + e], lane);
+        nj = h;
+        j0 += up * h;
+    } else if constexpr (S < LJ + LI) {
+        constexpr int h = M2 >> (S - LJ + 1);
+#pragma unroll
+        for (int i = 0; i < h; ++i)
+#pragma unroll
+            for (int e = 0; e < N; ++e)
+                acc[i * M1 * N + e] = lane_halve<S>(acc[i * M1 * N + e], acc[(i + h) * M1 * N + e], lane);
+        ni = h;
+        i0 += up * h;
+    } else {
+#pragma unroll
+        for (int e = 0; e < N; ++e) acc[e] = lane_full<S>(acc[e], lane);
+        first = first && !up;
+    }
+    if constexpr (S < 5) lane_reduce<M2, M1, N, S + 1>(acc, ls, lane, i0, ni, j0, nj, first);
+}
+
 // Segment kernel for the light classes (J/K modes): one block per segment of
 // a bra row, so every item of the block shares the bra pair (a b|.  The
 // exchange contributions of a quartet all land in the rows of the two bra
@@ -713,9 +795,13 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-template <int LA, int LB, int LC, int LD, int MODE>
+// SHARE: the form for lists in which some segments share items between
+// lanes; without it every item has one lane.
+template <int LA, int LB, int LC, int LD, int MODE, bool SHARE>
 __global__ void __launch_bounds__(256) k_eri_seg(EriArgs g) {
     constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
+    constexpr int NE = ((LA + LB + 1) * (LA + LB + 2) * (LA + LB + 3) - LA * (LA + 1) * (LA + 2)) / 6;
+    constexpr int NF = ((LC + LD + 1) * (LC + LD + 2) * (LC + LD + 3) - LC * (LC + 1) * (LC + 2)) / 6;
     using real = typename std::conditional<MODE == MODE_JK32, float, double>::type;
     extern __shared__ double seg_lds[];
     const int n = g.nbf;
@@ -740,35 +826,52 @@ __global__ void __launch_bounds__(256) k_eri_seg(EriArgs g) {
 #pragma unroll
         for (int i = 0; i < NA * NB; ++i) jab[i] = 0.0;
         const bool screen = g.dtol > 0.0;
-        for (long long t0 = seg.t0; t0 < seg.t0 + seg.n; t0 += blockDim.x) {
-            const long long t = t0 + threadIdx.x;
-            int pos = 0, b = 0, kp = 0;
+        const int ls = SHARE ? seg.ls : 0, ipw = 64 >> ls, sub = SHARE ? lane >> (6 - ls) : 0;
+        const int slot = SHARE ? (threadIdx.x >> 6) * ipw + (lane & (ipw - 1)) : threadIdx.x;
+        for (long long t0 = seg.t0; t0 < seg.t0 + seg.n; t0 += blockDim.x >> ls) {
+            const long long t = t0 + slot;
             bool live = t < seg.t0 + seg.n;
-            if (live) {
-                decode_in_row(g, seg.row, t, pos, b);
-                kp = g.ket_ids[pos];
-                if (screen) {
-                    const int2 ab = g.psh[bp], cd = g.psh[kp];
-                    const size_t ns = g.nsh, a = ab.x, bb = ab.y, c = cd.x, d = cd.y;
-                    double m = fmax(g.dsh[c * ns + d], g.dsh[a * ns + bb]);
-                    m = fmax(m, fmax(g.dsh[bb * ns + d], g.dsh[bb * ns + c]));
-                    m = fmax(m, fmax(g.dsh[a * ns + d], g.dsh[a * ns + c]));
-                    live = g.Qs[bp] * g.Qs[kp] * m >= g.dtol;
-                }
+            if (!SHARE && !screen && !live) continue;
+            int pos, b;
+            decode_in_row(g, seg.row, live ? t : seg.t0, pos, b);
+            const int kp = g.ket_ids[pos];
+            if (screen && live) {
+                const int2 ab = g.psh[bp], cd = g.psh[kp];
+                const size_t ns = g.nsh, a = ab.x, bb = ab.y, c = cd.x, d = cd.y;
+                double m = fmax(g.dsh[c * ns + d], g.dsh[a * ns + bb]);
+                m = fmax(m, fmax(g.dsh[bb * ns + d], g.dsh[bb * ns + c]));
+                m = fmax(m, fmax(g.dsh[a * ns + d], g.dsh[a * ns + c]));
+                live = g.Qs[bp] * g.Qs[kp] * m >= g.dtol;
             }
             if (screen) {
-                const unsigned long long mask = __ballot(live);
+                const unsigned long long mask = __ballot(live && sub == 0);
                 if (lane == 0 && mask) atomicAdd(g.kept, (unsigned)__popcll(mask));
             }
-            if (!live) continue;
-            const PairMeta mk = g.meta[kp];
-            const int fc = mk.fa, fd = mk.fb;
+            if ((!SHARE || ls == 0) && !live) continue;   // with shared items every lane takes part in the sums
+            const int nkp = !SHARE || live ? g.meta[kp].nprim : 0;
             const SoaKet kv{g.ksoa + g.bucket_soa[b] + (pos - g.bucket_start[b]),
                             g.bucket_start[b + 1] - g.bucket_start[b], g.kfs};
+            real acc[NE * NF];
+#pragma unroll
+            for (int i = 0; i < NE * NF; ++i) acc[i] = real(0);
+            for (int p = 0; p < mb.nprim; ++p) {
+                const PrimPair bq = bra[p];
+                for (int q = sub; q < nkp; q += 1 << ls)
+                    prim_vrr<real, LA, LB, LC, LD>(bq, kv.load(q), g.boysA, acc);
+            }
+            if constexpr (SHARE) {
+                if (ls) {
+                    int i0 = 0, ni = 1, j0 = 0, nj = 1;
+                    lane_reduce<1, 1, NE * NF>(acc, ls, lane, i0, ni, j0, nj, live);
+                    if (!live) continue;
+                }
+            }
+            const PairMeta mk = g.meta[kp];
+            const int fc = mk.fa, fd = mk.fb;
             real v[NA * NB * NC * ND];
             StoreCb<NB, NC, ND, real> st{v};
-            quartet<real, LA, LB, LC, LD>(bra, mb.nprim, kv, mk.nprim, ABx, ABy, ABz, g.ab[4 * kp],
-                                          g.ab[4 * kp + 1], g.ab[4 * kp + 2], g.boysA, st);
+            ClassCode<LA, LB, LC, LD, real>::hrr((real)ABx, (real)ABy, (real)ABz, (real)g.ab[4 * kp],
+                                                 (real)g.ab[4 * kp + 1], (real)g.ab[4 * kp + 2], acc, st);
             RegDigest<NA, NB, NC, ND, real> cb;
             cb.load(g.D, n, fa, fb, fc, fd);
 #pragma unroll
@@ -847,6 +950,11 @@ __device__ __forceinline__ double gc_dmax(const EriArgs& g, int x0, int x1, int 
     return m;
 }
 
+// The j-th member bound (a select: j differs between lanes).
+__device__ __forceinline__ double gc_pick(const double (&q)[4], int j) {
+    return j == 0 ? q[0] : j == 1 ? q[1] : j == 2 ? q[2] : q[3];
+}
+
 // With density screening (dtol > 0) an item is skipped when the group
 // bound (largest member Q of each side times the largest density block over
 // the groups' shells) is below dtol, and a member quartet is digested only
@@ -858,7 +966,7 @@ __device__ __forceinline__ double gc_dmax(const EriArgs& g, int x0, int x1, int 
 // TS: each member quartet's integrals are written to the ERI tensor g.out
 // (TensorCb, layout g.tpack) instead of digested; no LDS rows, no J/K.
 template <int LA, int LC, bool BT, bool TS = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LA == 1 && LC == 0 ? 3 : 1)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LA + LC < 2 ? 3 : 2)))
 k_eri_gc(EriArgs g) {
     constexpr int NA = ncart(LA), NC = ncart(LC), NI = NA * NC;
     constexpr int MB = LA == 0 ? 4 : 2, MK = LC == 0 ? 4 : 2;
@@ -899,14 +1007,16 @@ k_eri_gc(EriArgs g) {
         for (int i = 0; i < MB * NA; ++i) jab[i] = 0.0;
         const bool screen = g.dtol > 0.0;
         unsigned nkept = 0;
-        for (long long t0 = seg.t0; t0 < seg.t0 + seg.n; t0 += blockDim.x) {
-            const long long t = t0 + threadIdx.x;
-            if (t >= seg.t0 + seg.n) continue;
+        const int ls = seg.ls, ipw = 64 >> ls, sub = lane >> (6 - ls);
+        const int slot = (threadIdx.x >> 6) * ipw + (lane & (ipw - 1));
+        for (long long t0 = seg.t0; t0 < seg.t0 + seg.n; t0 += blockDim.x >> ls) {
+            const long long t = t0 + slot;
+            bool live = t < seg.t0 + seg.n;
             int pos, b;
-            decode_in_row(g, seg.row, t, pos, b);
+            decode_in_row(g, seg.row, live ? t : seg.t0, pos, b);
             const int kp = g.ket_ids[pos];
-            const GcMeta mk = g.gmeta[kp];
-            if (screen) {
+            if (screen && live) {
+                const GcMeta mk = g.gmeta[kp];
                 double qb = 0.0, qk = 0.0;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) { qb = fmax(qb, mb.q[i]); qk = fmax(qk, mk.q[i]); }
@@ -916,8 +1026,10 @@ k_eri_gc(EriArgs g) {
                 m = fmax(m, gc_dmax(g, mb.sb0, mb.sb1, mk.sa0, mk.sa1));
                 m = fmax(m, gc_dmax(g, mb.sa0, mb.sa1, mk.sb0, mk.sb1));
                 m = fmax(m, gc_dmax(g, mb.sa0, mb.sa1, mk.sa0, mk.sa1));
-                if (qb * qk * m < g.dtol) continue;
+                live = qb * qk * m >= g.dtol;
             }
+            if (ls == 0 && !live) continue;       // with shared items every lane takes part in the sums
+            const int nkp = live ? g.gmeta[kp].nprim : 0;
             const int nk = g.bucket_start[b + 1] - g.bucket_start[b];
             const double* kb = g.ksoa + g.bucket_soa[b] + (pos - g.bucket_start[b]);
             double acc[MB * MK * NI];
@@ -925,7 +1037,7 @@ k_eri_gc(EriArgs g) {
             for (int i = 0; i < MB * MK * NI; ++i) acc[i] = 0.0;
             // ket primitive outer (its fields stay in registers), bra inner
             // (the same for the whole block: scalar loads)
-            for (int q = 0; q < mk.nprim; ++q) {
+            for (int q = sub; q < nkp; q += 1 << ls) {
                 const double* x = kb + (long long)q * nk;
                 PrimPair kq;
                 kq.zeta = x[0]; kq.K = x[fs]; kq.Px = x[2 * fs]; kq.Py = x[3 * fs]; kq.Pz = x[4 * fs];
@@ -980,12 +1092,23 @@ k_eri_gc(EriArgs g) {
                     }
                 }
             }
+            int i0 = 0, ni = MB, j0 = 0, nj = MK;
+            lane_reduce<MB, MK, NI>(acc, ls, lane, i0, ni, j0, nj, live);
+            if (!live) continue;
+            // both pairs' data again: keeping the bra's 28 scalars across the
+            // primitive loops spilled them
+            int kp2 = kp, bp2 = __builtin_amdgcn_readfirstlane(bp);
+            asm volatile("" : "+v"(kp2), "+s"(bp2));
+            const GcMeta mk = g.gmeta[kp2], mb = g.gmeta[bp2];
             const double sq = bp == kp ? 0.5 : 1.0;
-            // ket member outer: its J_cd block is summed over the bra members
-            // in registers and added once
+            // ket member outer: its J_cd block is summed over the lane's bra
+            // members in registers and added once
 #pragma unroll
-            for (int j = 0; j < MK; ++j) {
+            for (int jj = 0; jj < MK; ++jj) {
+                if (jj >= nj) break;
+                const int j = j0 + jj;
                 if (j >= mk.m) break;
+                const double qkj = gc_pick(mk.q, j);
                 const int kc = (mk.code >> (2 * j)) & 1, kd = (mk.code >> (2 * j + 1)) & 1;
                 const int fc = kc ? mk.fa1 : mk.fa0, fd = kd ? mk.fb1 : mk.fb0;
                 double jcd[NC];
@@ -993,9 +1116,12 @@ k_eri_gc(EriArgs g) {
                 for (int c = 0; c < NC; ++c) jcd[c] = 0.0;
                 bool any = false;
 #pragma unroll
-                for (int i = 0; i < MB; ++i) {
-                    if (i >= mb.m) break;
-                    if (mb.q[i] * mk.q[j] < g.qtol) continue;
+                for (int ii = 0; ii < MB; ++ii) {
+                    if (ii >= ni) break;
+                    const int i = i0 + ii;
+                    if (i >= mb.m) continue;
+                    const double qij = gc_pick(mb.q, i) * qkj;
+                    if (qij < g.qtol) continue;
                     const int ia = (mb.code >> (2 * i)) & 1, ib = (mb.code >> (2 * i + 1)) & 1;
                     const int fa = ia ? mb.fa1 : mb.fa0, fb = ib ? mb.fb1 : mb.fb0;
                     if (screen) {
@@ -1005,12 +1131,12 @@ k_eri_gc(EriArgs g) {
                         double m = fmax(g.dsh[c * ns + d], g.dsh[a * ns + bb]);
                         m = fmax(m, fmax(g.dsh[bb * ns + d], g.dsh[bb * ns + c]));
                         m = fmax(m, fmax(g.dsh[a * ns + d], g.dsh[a * ns + c]));
-                        if (mb.q[i] * mk.q[j] * m < g.dtol) continue;
+                        if (qij * m < g.dtol) continue;
                         nkept += bp != kp || j <= i;   // both orders of a bra == ket row are one quartet
                     }
                     double v[NI];
                     StoreCb<1, NC, 1, double> st{v};
-                    ClassCode<LA, 0, LC, 0, double>::hrr(0.0, 0.0, 0.0, 0.0, 0.0, 0.0, acc + (i * MK + j) * NI, st);
+                    ClassCode<LA, 0, LC, 0, double>::hrr(0.0, 0.0, 0.0, 0.0, 0.0, 0.0, acc + (ii * MK + jj) * NI, st);
                     if constexpr (TS) {
                         TensorCb tc{g.out, (size_t)n, fa, fb, fc, fd, g.tpack};
 #pragma unroll
@@ -1028,7 +1154,9 @@ k_eri_gc(EriArgs g) {
                     const double s = (fa == fb ? 0.5 : 1.0) * (fc == fd ? 0.5 : 1.0) * sq;
 #pragma unroll
                     for (int a = 0; a < NA; ++a) {
-                        jab[i * NA + a] += s * cb.Jab[a];
+                        // a lane of a shared item keeps other members than 0 .. ni - 1
+#pragma unroll
+                        for (int x = 0; x < MB; ++x) jab[x * NA + a] += x == i ? s * cb.Jab[a] : 0.0;
                         double* row = Kr + (size_t)(ia * NA + a) * n;
 #pragma unroll
                         for (int c = 0; c < NC; ++c) atomicAdd(&row[fc + c], s * cb.Kac[a * NC + c]);
@@ -1169,15 +1297,17 @@ __global__ void __launch_bounds__(256) k_eri_gck(EriArgs g) {
 #pragma unroll
         for (int i = 0; i < NA * NB; ++i) jab[i] = 0.0;
         unsigned nkept = 0;
-        for (long long t0 = seg.t0; t0 < seg.t0 + seg.n; t0 += blockDim.x) {
-            const long long t = t0 + threadIdx.x;
-            if (t >= seg.t0 + seg.n) continue;
+        const int ls = seg.ls, ipw = 64 >> ls, sub = lane >> (6 - ls);
+        const int slot = (threadIdx.x >> 6) * ipw + (lane & (ipw - 1));
+        for (long long t0 = seg.t0; t0 < seg.t0 + seg.n; t0 += blockDim.x >> ls) {
+            const long long t = t0 + slot;
+            bool live = t < seg.t0 + seg.n;
             int pos, b;
-            decode_in_row(g, seg.row, t, pos, b);
+            decode_in_row(g, seg.row, live ? t : seg.t0, pos, b);
             const int kp = g.ket_ids[pos];
-            const GcMeta mk = g.gmeta[kp];
             const int2 ab = screen ? g.psh[bp] : make_int2(0, 0);
-            if (screen) {
+            if (screen && live) {
+                const GcMeta mk = g.gmeta[kp];
                 double qk = 0.0;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) qk = fmax(qk, mk.q[i]);
@@ -1187,14 +1317,16 @@ __global__ void __launch_bounds__(256) k_eri_gck(EriArgs g) {
                 m = fmax(m, gc_dmax(g, ab.y, -1, mk.sa0, mk.sa1));
                 m = fmax(m, gc_dmax(g, ab.x, -1, mk.sb0, mk.sb1));
                 m = fmax(m, gc_dmax(g, ab.x, -1, mk.sa0, mk.sa1));
-                if (qb * qk * m < g.dtol) continue;
+                live = qb * qk * m >= g.dtol;
             }
+            if (ls == 0 && !live) continue;       // with shared items every lane takes part in the sums
+            const int nkp = live ? g.gmeta[kp].nprim : 0;
             const int nk = g.bucket_start[b + 1] - g.bucket_start[b];
             const double* kb = g.ksoa + g.bucket_soa[b] + (pos - g.bucket_start[b]);
             double acc[MK * NE * NF];
 #pragma unroll
             for (int i = 0; i < MK * NE * NF; ++i) acc[i] = 0.0;
-            for (int q = 0; q < mk.nprim; ++q) {
+            for (int q = sub; q < nkp; q += 1 << ls) {
                 const double* x = kb + (long long)q * nk;
                 PrimPair kq;
                 kq.zeta = x[0]; kq.K = x[fs]; kq.Px = x[2 * fs]; kq.Py = x[3 * fs]; kq.Pz = x[4 * fs];
@@ -1210,27 +1342,34 @@ __global__ void __launch_bounds__(256) k_eri_gck(EriArgs g) {
                     for (int e = 0; e < NE * NF; ++e) acc[j * NE * NF + e] += wk * sb[e];
                 }
             }
-            // one digestion instance: member j is always in acc[0 ..), the
-            // accumulators move down one member after each step
+            int i0 = 0, ni = 1, j0 = 0, nj = MK;
+            lane_reduce<1, MK, NE * NF>(acc, ls, lane, i0, ni, j0, nj, live);
+            if (!live) continue;
+            const GcMeta mk = g.gmeta[kp];
+            // one digestion instance: the lane's next member is always in
+            // acc[0 ..), the accumulators move down one member after each step
 #pragma unroll 1
-            for (int j = 0; j < mk.m; ++j) {
+            for (int jj = 0; jj < nj; ++jj) {
+                const int j = j0 + jj;
+                if (j >= mk.m) break;
+                const double qkj = gc_pick(mk.q, j);
                 const int kc = (mk.code >> (2 * j)) & 1, kd = (mk.code >> (2 * j + 1)) & 1;
                 const int fc = kc ? mk.fa1 : mk.fa0, fd = kd ? mk.fb1 : mk.fb0;
-                bool live = qb * mk.q[j] >= g.qtol;
-                if (screen && live) {
+                bool keep = qb * qkj >= g.qtol;
+                if (screen && keep) {
                     const size_t ns = g.nsh;
                     const int c = kc ? mk.sa1 : mk.sa0, d = kd ? mk.sb1 : mk.sb0;
                     double m = fmax(g.dsh[c * ns + d], g.dsh[ab.x * ns + ab.y]);
                     m = fmax(m, fmax(g.dsh[ab.y * ns + d], g.dsh[ab.y * ns + c]));
                     m = fmax(m, fmax(g.dsh[ab.x * ns + d], g.dsh[ab.x * ns + c]));
-                    live = qb * mk.q[j] * m >= g.dtol;
-                    nkept += live;
+                    keep = qb * qkj * m >= g.dtol;
+                    nkept += keep;
                 }
-                if (live) gck_digest<LA, LB, LC>(g, acc, ABx, ABy, ABz, fa, fb, fc, fd, Kr, J, jab);
+                if (keep) gck_digest<LA, LB, LC>(g, acc, ABx, ABy, ABz, fa, fb, fc, fd, Kr, J, jab);
 #pragma unroll
-                for (int jj = 0; jj + 1 < MK; ++jj)
+                for (int x = 0; x + 1 < MK; ++x)
 #pragma unroll
-                    for (int e = 0; e < NE * NF; ++e) acc[jj * NE * NF + e] = acc[(jj + 1) * NE * NF + e];
+                    for (int e = 0; e < NE * NF; ++e) acc[x * NE * NF + e] = acc[(x + 1) * NE * NF + e];
             }
         }
 #pragma unroll
@@ -1260,8 +1399,9 @@ __global__ void __launch_bounds__(256) k_eri_gck(EriArgs g) {
 
 typedef void (*EriKernel)(EriArgs);
 // Getter modes of polyeri_class_kernel beyond the k_eri modes: the segment
-// kernel for MODE_JK and MODE_JK32.
-enum { GET_SEG_JK = 5, GET_SEG_JK32 = 6 };
+// kernel for MODE_JK and MODE_JK32, and for MODE_JK with items shared between
+// lanes.
+enum { GET_SEG_JK = 5, GET_SEG_JK32 = 6, GET_SEG_SHARE = 7 };
 // Strided batched FP64 products on the MFMA units (kgemm.hip):
 // C_b(m,n) = sum_k A_b(m,k) B_b(k,n), X_b(r,c) = X[b*sX + r*sXr + c*sXc].
 enum { GEMM_F64 = 1, GEMM_BF16X3 = 2 };

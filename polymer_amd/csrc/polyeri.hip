@@ -282,60 +282,87 @@ static const int RYS_NMAX_EXPORT = 5;
 static const int kSegItems = 2048, kSegMin = 256;
 static const double kSegTarget = 4096.0;
 
+// Lanes (log2) that share one item of bp bra and kp ket primitive pairs.  One
+// lane per item makes the longest chain of a deeply contracted basis, 81 x 81
+// primitive quartets for two oxygen 1s/2s group pairs of cc-pVDZ, the length
+// of the whole launch: k_eri_gc (ss|ss) took 1.62 ms for one water and 1.94
+// for nine.  Sharing costs the sums over the lanes and, where an item has one
+// member, a digestion on one lane in 2^ls.  So a chain may be as long as half
+// of what each lane of the full chip (kSplitLanes: two wavefronts a SIMD)
+// does for the list; a shorter one is shared while it exceeds a sixteenth of
+// what a lane does for all lists, which run side by side and hide each
+// other's ends, held between kSplitMin and kSplitMax primitive quartets (from
+// about one digestion's time to several).  In a large build only the longest
+// items are shared, in a small one, whose lanes are idle, nearly all.
+static const double kSplitLanes = 256.0 * 4 * 64 * 2, kSplitMin = 8.0, kSplitMax = 128.0;
+static int segment_split(double bp, double kp, double list_total, double ctx_total) {
+    const double limit = std::max(0.5 * list_total / kSplitLanes,
+                                  std::min(std::max(ctx_total / kSplitLanes / 16.0, kSplitMin), kSplitMax));
+    int ls = 0;
+    while (ls < 6 && (1 << ls) < kp && bp * kp > limit * (1 << ls)) ++ls;
+    return ls;
+}
+
 // Bra-row segments of a work list for the segment kernels: each segment is
 // part of one row, at most kSegItems items and about `target` primitive
 // quartets (the row's bra primitive count times each ket's), with target =
-// the list's primitive quartets / kSegTarget, but at least kSegMin items (one
-// pass of a block: shorter segments pay more for their row flush than they
-// gain in balance) where the row has them; ordered by
+// the list's primitive quartets / kSegTarget, but at least one pass of a
+// block (kSegMin lanes: shorter segments pay more for their row flush than
+// they gain in balance) where the row has them; ordered by
 // primitive quartets, largest first, so that the blocks launched last are
-// the short ones.  pairs / bra / kets / bstart: the list's pair data, bra
-// ids by row, ket ids and bucket starts of the ket class.  balanced = false:
-// rows cut every kSegItems items, in row order (the autotuner keeps
-// whichever form is faster per list).
+// the short ones.  The items of a segment are shared by equally many lanes
+// (segment_split; split = the primitive quartets of all lists, 0: one lane
+// each), so a row is also cut where that changes.  pairs / bra / kets /
+// bstart: the list's pair data, bra ids by row, ket ids and bucket starts of
+// the ket class.  balanced = false: rows cut every kSegItems lanes, in row
+// order (the autotuner keeps whichever form is faster per list).
 static std::vector<SegDesc> make_segments(const WorkList& l, const std::vector<PairInfo>& pairs,
                                           const std::vector<int>& bra, const std::vector<int>& kets,
-                                          const std::vector<int>& bstart, bool balanced = true) {
+                                          const std::vector<int>& bstart, double split, bool balanced = true) {
     const int nb = l.nbucket;
-    if (!balanced) {
-        std::vector<SegDesc> out;
-        for (int r = 0; r < l.nrows; ++r)
-            for (long long t = l.row[r]; t < l.row[r + 1]; t += kSegItems)
-                out.push_back(SegDesc{t, r, (int)std::min<long long>(kSegItems, l.row[r + 1] - t)});
-        return out;
-    }
     std::vector<double> knp(nb, 0.0);
     for (int b = 0; b + 1 < (int)bstart.size() && b < nb; ++b) knp[b] = pairs[kets[bstart[b]]].nprim;
-    const double target = l.prim_quartets / kSegTarget;
+    const double target = balanced ? l.prim_quartets / kSegTarget : 1e300;
     std::vector<std::pair<double, SegDesc>> segs;
     for (int r = 0; r < l.nrows; ++r) {
         const double bp = pairs[bra[r]].nprim;
         const int* rb = l.rb.data() + (size_t)r * (nb + 1);
         long long t = l.row[r];
-        int n = 0;
+        int n = 0, ls = 0;
         double cost = 0.0;
+        auto flush = [&] {
+            if (n > 0) segs.push_back({cost, SegDesc{t, r, n, ls}});
+            t += n; n = 0; cost = 0.0;
+        };
         for (int b = 0; b < nb; ++b) {
             int cnt = rb[b + 1] - rb[b];
+            if (cnt <= 0) continue;
             const double ci = bp * knp[b];
+            const int lb = split > 0.0 ? segment_split(bp, knp[b], l.prim_quartets, split) : 0;
+            if (lb != ls) flush();
+            ls = lb;
+            const int nmax = kSegItems >> ls, nmin = kSegMin >> ls;
             while (cnt > 0) {
-                int take = std::min(cnt, kSegItems - n);
+                int take = std::min(cnt, nmax - n);
                 if (ci > 0.0)
-                    take = (int)std::min<double>(take, std::max<double>(kSegMin - n, std::ceil((target - cost) / ci)));
+                    take = (int)std::min<double>(take, std::max<double>(nmin - n, std::ceil((target - cost) / ci)));
                 take = std::max(take, 1);
                 n += take; cost += take * ci; cnt -= take;
-                if (n >= kSegItems || (n >= kSegMin && cost >= target)) {
-                    segs.push_back({cost, SegDesc{t, r, n}});
-                    t += n; n = 0; cost = 0.0;
-                }
+                if (n >= nmax || (n >= nmin && cost >= target)) flush();
             }
         }
-        if (n > 0) segs.push_back({cost, SegDesc{t, r, n}});
+        flush();
     }
-    std::stable_sort(segs.begin(), segs.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
+    if (balanced)
+        std::stable_sort(segs.begin(), segs.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
     std::vector<SegDesc> out(segs.size());
     for (size_t i = 0; i < segs.size(); ++i) out[i] = segs[i].second;
     return out;
 }
+static bool shares_items(const std::vector<SegDesc>& segs) {
+    return std::any_of(segs.begin(), segs.end(), [](const SegDesc& s) { return s.ls > 0; });
+}
+
 // Largest ket Schwarz bound kq over the items of each segment.  A row's
 // items cover one contiguous range of ket positions per bucket (the
 // decode_in_row mapping), so a sparse table of range maxima over the ket
@@ -393,6 +420,7 @@ struct ClassPairWork {
     SegDesc* d_seg;        // bra-row segments (molecular lists): nseg cost-balanced ones, then
     int nseg, nsegc;       // nsegc of kSegItems items each (make_segments)
     double* d_segq;        // per segment of d_seg: the largest ket bound (segment_ket_bounds)
+    bool share[2];         // whether some of the nseg (nsegc) segments share items between lanes
     LaunchCfg cfg;         // launch shape (autotuned or default)
     int prec;              // 0: FP64, 1: FP32 (mixed precision)
     int both;              // periodic lists of two different classes: both bra/ket roles
@@ -612,7 +640,7 @@ static int launch_class(polyeri_ctx* c, int mode, int la, int lb, int lc, int ld
                         const int* rb = nullptr, const int* bstart = nullptr, int nbucket = 0,
                         const int* rf = nullptr, const int2* items = nullptr, const unsigned* count = nullptr,
                         LaunchCfg cfg = LaunchCfg(), const int* bsoa = nullptr, const SegDesc* segs = nullptr,
-                        int nseg = 0, const SegScreen* scr = nullptr) {
+                        int nseg = 0, const SegScreen* scr = nullptr, bool share = false) {
     if (nwork <= 0) return 0;
     EriArgs a{};
     a.ksoa = c->d_ksoa; a.kfs = (long long)c->prims.size(); a.bucket_soa = bsoa;
@@ -662,7 +690,8 @@ static int launch_class(polyeri_ctx* c, int mode, int la, int lb, int lc, int ld
         }
     }
     if (kind == LAUNCH_SEG) {
-        EriKernel ks = polyeri_class_kernel(la, lb, lc, ld, mode == MODE_JK ? GET_SEG_JK : GET_SEG_JK32);
+        EriKernel ks = polyeri_class_kernel(
+            la, lb, lc, ld, mode != MODE_JK ? GET_SEG_JK32 : share ? GET_SEG_SHARE : GET_SEG_JK);
         if (!ks) return fail(POLYERI_E_ARG, "no segment kernel for class");
         a.segs = segs;
         a.nseg = nseg;
@@ -982,8 +1011,8 @@ static int build_gc_lists(polyeri_ctx* c) {
         for (ClassPairWork& x : c->work)
             if (x.X == l.X && x.Y == l.Y && x.prec == 0) w = &x;
         if (!w) continue;
-        std::vector<SegDesc> segs = make_segments(l, gp, cls[l.X], kets[l.Y], bst[l.Y]);
-        const std::vector<SegDesc> segc = make_segments(l, gp, cls[l.X], kets[l.Y], bst[l.Y], false);
+        std::vector<SegDesc> segs = make_segments(l, gp, cls[l.X], kets[l.Y], bst[l.Y], c->prim_quartets);
+        const std::vector<SegDesc> segc = make_segments(l, gp, cls[l.X], kets[l.Y], bst[l.Y], c->prim_quartets, false);
         if (segs.size() + segc.size() > 0x7fffffffu) return fail(POLYERI_E_ARG, "too many segments");
         auto& g = w->gc;
         g.nwork = l.nwork; g.nrows = l.nrows; g.nbucket = l.nbucket;
@@ -1035,8 +1064,8 @@ static int build_gc_lists(polyeri_ctx* c) {
         for (ClassPairWork& x : c->work)
             if (x.X == l.X && x.Y == l.Y && x.prec == 0) w = &x;
         if (!w || w->gc.nwork > 0) continue;
-        std::vector<SegDesc> segs = make_segments(l, cp, cid[l.X], ck[l.Y], cb[l.Y]);
-        const std::vector<SegDesc> segc = make_segments(l, cp, cid[l.X], ck[l.Y], cb[l.Y], false);
+        std::vector<SegDesc> segs = make_segments(l, cp, cid[l.X], ck[l.Y], cb[l.Y], c->prim_quartets);
+        const std::vector<SegDesc> segc = make_segments(l, cp, cid[l.X], ck[l.Y], cb[l.Y], c->prim_quartets, false);
         if (segs.size() + segc.size() > 0x7fffffffu) return fail(POLYERI_E_ARG, "too many segments");
         auto& g = w->gc;
         g.kind = 1;
@@ -1215,6 +1244,8 @@ static int build_ctx(polyeri_ctx* c) {
         HIPCHK(hipMemcpy(c->d_ksoa, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice));
     }
     c->quartets = 0; c->prim_quartets = 0; c->model_flops = 0;
+    double all = 0.0;
+    for (const WorkList& l : wl) all += l.prim_quartets;
     for (const WorkList& l : wl) {
         ClassPairWork w;
         w.X = l.X; w.Y = l.Y;
@@ -1231,6 +1262,7 @@ static int build_ctx(polyeri_ctx* c) {
         w.d_seg = nullptr;
         w.d_segq = nullptr;
         w.nseg = w.nsegc = 0;
+        w.share[0] = w.share[1] = false;
         w.prim_quartets = l.prim_quartets;
         w.flops = l.prim_quartets * flop_model(w.la, w.lb, w.lc, w.ld);
         w.d_row = nullptr;
@@ -1247,13 +1279,17 @@ static int build_ctx(polyeri_ctx* c) {
         // stays in bounds), so it is not launched, and mixed contexts do not
         // split the light classes.
         if (!c->pbc && l.nwork > 0 && (!l.prec || polyeri_rys_class(w.la, w.lb, w.lc, w.ld))) {
+            // the Rys kernel has its own lanes per item
+            const double split = polyeri_rys_class(w.la, w.lb, w.lc, w.ld) ? 0.0 : all;
             std::vector<SegDesc> segs =
-                make_segments(l, c->pairs, c->class_ids[l.X], c->ket_ids[l.Y], c->bstart[l.Y]);
+                make_segments(l, c->pairs, c->class_ids[l.X], c->ket_ids[l.Y], c->bstart[l.Y], split);
             const std::vector<SegDesc> segc =
-                make_segments(l, c->pairs, c->class_ids[l.X], c->ket_ids[l.Y], c->bstart[l.Y], false);
+                make_segments(l, c->pairs, c->class_ids[l.X], c->ket_ids[l.Y], c->bstart[l.Y], split, false);
             if (segs.size() + segc.size() > 0x7fffffffu) return fail(POLYERI_E_ARG, "too many segments");
             w.nseg = (int)segs.size();
             w.nsegc = (int)segc.size();
+            w.share[0] = shares_items(segs);
+            w.share[1] = shares_items(segc);
             segs.insert(segs.end(), segc.begin(), segc.end());
             if ((rc = dalloc(&w.d_seg, segs.size()))) return rc;
             HIPCHK(hipMemcpy(w.d_seg, segs.data(), segs.size() * sizeof(SegDesc), hipMemcpyHostToDevice));
@@ -1488,7 +1524,8 @@ int polyeri_autotune(polyeri_ctx* ctx, int reps) {
                 if (r == 1) HIPCHK(hipEventRecord(e0, c->stream));
                 rc = launch_class(c, mode, cw.la, cw.lb, cw.lc, cw.ld, cw.d_bra, cw.d_ket, cw.d_row, cw.nrows,
                                   cw.nwork, nullptr, cw.d_rb, cw.d_bstart, cw.nbucket, cw.d_rf, nullptr, nullptr, x,
-                                  cw.d_bsoa, x.segv ? cw.d_seg + cw.nseg : cw.d_seg, x.segv ? cw.nsegc : cw.nseg);
+                                  cw.d_bsoa, x.segv ? cw.d_seg + cw.nseg : cw.d_seg, x.segv ? cw.nsegc : cw.nseg,
+                                  nullptr, cw.share[x.segv ? 1 : 0]);
             }
             if (rc) break;
             HIPCHK(hipEventRecord(e1, c->stream));
@@ -1705,7 +1742,8 @@ static int jk_enqueue(polyeri_ctx* c, const double* d_pc, double* d_jc, double* 
                               cw.d_row, cw.nrows, cw.nwork, nullptr, cw.d_rb, cw.d_bstart, cw.nbucket, cw.d_rf,
                               screen && !seg ? cw.d_items : nullptr, screen && !seg ? c->d_counts + w : nullptr,
                               cw.cfg, cw.d_bsoa, cw.cfg.segv ? cw.d_seg + cw.nseg : cw.d_seg,
-                              cw.cfg.segv ? cw.nsegc : cw.nseg, screen && seg ? &scr : nullptr);
+                              cw.cfg.segv ? cw.nsegc : cw.nseg, screen && seg ? &scr : nullptr,
+                              cw.share[cw.cfg.segv ? 1 : 0]);
         }
         c->stream = main;
     }

@@ -1,0 +1,49 @@
+"""Work items shared between the lanes of a wavefront (segment and generally
+contracted J/K kernels): the ket primitive pairs of a deeply contracted item
+are divided over 2 .. 64 lanes and summed back.  Small molecules share nearly
+every item, so the cases below reach every lane count, lists shorter than a
+wavefront, ket counts that are not a multiple of the lanes, and one member
+(shell pairs) or several (s-shell groups) an item."""
+import numpy as np
+import pytest
+
+import oracle
+import polymer_amd as pa
+from tests.conftest import basis_path
+from tests.molecules import BH_GOLDEN, H2O_GOLDEN
+
+pytestmark = pytest.mark.gpu
+
+CASES = {
+    "ne_ccpvdz": ([(10, 0.1, 0.0, -0.2)], "cc-pVDZ"),
+    "h2o_ccpvdz": (H2O_GOLDEN, "cc-pVDZ"),
+    "h2o_631g": (H2O_GOLDEN, "6-31G"),
+    "h2_631gss": ([(1, 0.0, 0.0, 0.0), (1, 0.0, 0.0, 1.4)], "6-31Gss"),
+    "bh_sto3g": (BH_GOLDEN, "STO-3G"),
+}
+
+
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("grouped", [True, False])
+def test_shared_items_match_oracle(case, grouped):
+    """J/K at Schwarz 0 against the oracle, and the density-screened form at a
+    threshold below every bound, which has to keep every quartet.  Tolerance:
+    sums of at most 10^5 terms below 10 in FP64, 10^5 x 10 x 2^-53 = 1e-10."""
+    atoms, basis = CASES[case]
+    b = pa.read_basis(basis, atoms)
+    rng = np.random.default_rng(7)
+    real = b.real_functions
+    p = np.zeros((b.ncgs, b.ncgs))
+    a = 0.1 * rng.standard_normal((len(real), len(real)))
+    p[np.ix_(real, real)] = a + a.T
+    ctx = pa.Context(b, schwarz_tol=0.0)
+    ctx.set_general_contraction(grouped)
+    print(f"case: shared items {case} grouped {grouped}", flush=True)
+    j, k = ctx.fourindex_eri(p)
+    n = ctx.stats()["last_quartets"]
+    jr, kr = oracle.Basis(basis_path(basis), atoms).fourindex_eri(p, 0.0)[:2]
+    assert np.max(np.abs(jr)) > 0 and np.max(np.abs(kr)) > 0
+    assert np.max(np.abs(j - jr)) < 1e-10 and np.max(np.abs(k - kr)) < 1e-10
+    js, ks = ctx.fourindex_eri(p, dens_tol=1e-290)
+    assert np.max(np.abs(js - jr)) < 1e-10 and np.max(np.abs(ks - kr)) < 1e-10
+    assert ctx.stats()["last_quartets"] >= n       # every quartet kept
