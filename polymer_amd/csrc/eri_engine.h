@@ -26,30 +26,32 @@
 #define BOYS_NT 801
 #define BOYS_NM 16
 #define BOYS_TMAX 40.0
-// The thread kernels read a second layout of the same values: for each
-// L < BOYS_LA a table of 64-byte rows F_L(T_i) .. F_{L+6}(T_i) (and one pad),
-// so the seven values of one lookup arrive in four 16-byte loads.  It follows
-// the BOYS_NT x BOYS_NM table in the same allocation (BOYS_AOFF doubles in).
+// The thread kernels read a second layout: Taylor coefficients of the lower
+// of the two orders a lookup returns, F_{l+k}(T_i) / k! (k = 0..7, l = L - 1,
+// or 0 for L = 0), one 64-byte row per L < BOYS_LA and grid point, so a
+// lookup is four 16-byte loads.  It follows the BOYS_NT x BOYS_NM table in
+// the same allocation (BOYS_AOFF doubles in).
 #define BOYS_LA 9
 #define BOYS_AOFF (BOYS_NT * BOYS_NM)
 // A third layout, small enough for LDS, for the kernels that copy it there:
-// for each L < BOYS_LC, rows F_L(T_j) .. F_{L+9}(T_j) on the coarse grid
-// T_j = j/5 (every fourth point of the main grid), j = 0..BOYS_CNT-1, read
-// with a ten-term Taylor step (|h| <= 0.1, truncation below 1e-18).  It
-// follows the aligned tables (BOYS_COFF doubles in); BOYS_CROWS doubles
-// (16 080 bytes) per L.
+// for each L < BOYS_LC, rows of ten coefficients F_{l+k}(T_j) / k! on the
+// coarse grid T_j = 3 j / 20 (every third point of the main grid; the last
+// row also serves T up to BOYS_TMAX).  |h| <= 0.075 leaves less than 3e-17 of
+// the result.  It follows the aligned tables (BOYS_COFF doubles in);
+// BOYS_CROWS doubles (21 360 bytes) per L.
 #define BOYS_LC 7
-#define BOYS_CNT 201
+#define BOYS_CNT 267
 #define BOYS_CROWS (BOYS_CNT * 10)
 #define BOYS_COFF (BOYS_AOFF + BOYS_LA * BOYS_NT * 8)
 
 // Primitive pair of a shell pair (a,b): exponent sum, prefactor with both
-// contraction coefficients, centre P and P - A.  64 bytes.
+// contraction coefficients, centre P, P - A and 1 / (2 zeta).
 struct PrimPair {
     double zeta;
     double K;   // c_a c_b sqrt(2) pi^{5/4} exp(-ab/zeta |AB|^2) / zeta
     double Px, Py, Pz;
     double PAx, PAy, PAz;
+    double h;   // 1 / (2 zeta): stored, a division costs ten FP64 instructions a primitive quartet
 };
 
 // Generally contracted pair (classes (ls|), s shells that share exponents):
@@ -118,19 +120,65 @@ struct SoaKet {
         const double* x = p + (long long)q * nk;
         PrimPair r;
         r.zeta = x[0]; r.K = x[fs]; r.Px = x[2 * fs]; r.Py = x[3 * fs]; r.Pz = x[4 * fs];
-        r.PAx = x[5 * fs]; r.PAy = x[6 * fs]; r.PAz = x[7 * fs];
+        r.PAx = x[5 * fs]; r.PAy = x[6 * fs]; r.PAz = x[7 * fs]; r.h = x[8 * fs];
         return r;
     }
 };
 
-// F_0..F_L (T) scaled by pref.  FP64: 7-term Taylor step for F_L around the
-// nearest grid point, then the downward recursion
-// F_{m-1} = (2T F_m + e^-T) / (2m-1); large T: asymptotic F_0 and the
-// upward recursion without the (negligible) e^-T term.
 // Two table values loaded as one 16-byte word.
 struct alignas(16) BoysPair {
     double x, y;
 };
+
+// F_0..F_L (T) scaled by pref.  Below BOYS_TMAX: the Taylor polynomial of
+// F_{L-1} around the nearest grid point and, by the same Horner loop, its
+// derivative, which is F_L (dF_m/dT = -F_{m+1} and h = T_i - T); then
+// e^-T = (2L - 1) F_{L-1} - 2T F_L, whose rounding error is below an ulp of
+// every sum it enters, and the downward recursion
+// F_{m-1} = (2T F_m + e^-T) / (2m-1).  (The recursion from F_L alone needs
+// exp(-T), about 28 FP64 instructions, more than the second polynomial and
+// the rest of the lookup.)  Above: the asymptotic F_0 and the upward
+// recursion without the (negligible) e^-T term.
+// N coefficients at c, grid distance h.
+template <int L, int N>
+POLY_HD void boys_rows(double T, double h, const double* __restrict__ c, double* __restrict__ F) {
+    const BoysPair* g = reinterpret_cast<const BoysPair*>(c);
+    double w[N];
+#pragma unroll
+    for (int k = 0; k < N / 2; ++k) {
+        const BoysPair p = g[k];
+        w[2 * k] = p.x;
+        w[2 * k + 1] = p.y;
+    }
+    double b = w[N - 1];
+    if constexpr (L == 0) {
+#pragma unroll
+        for (int k = N - 2; k >= 0; --k) b = __builtin_fma(b, h, w[k]);
+        F[0] = b;
+    } else {
+        double d = 0.0;
+#pragma unroll
+        for (int k = N - 2; k >= 0; --k) {
+            d = k == N - 2 ? b : __builtin_fma(d, h, b);
+            b = __builtin_fma(b, h, w[k]);
+        }
+        F[L] = d;
+        F[L - 1] = b;
+        if constexpr (L > 1) {
+            const double t2 = 2.0 * T;
+            const double e = __builtin_fma(2 * L - 1, b, -t2 * d);
+#pragma unroll
+            for (int m = L - 2; m >= 0; --m) F[m] = (t2 * F[m + 1] + e) * (1.0 / (2 * m + 1));
+        }
+    }
+}
+template <int L>
+POLY_HD void boys_large(double T, double* __restrict__ F) {
+    const double r = rsqrt_fp64(T), it = r * r;
+    F[0] = 0.5 * POLY_SQRT_PI * r;
+#pragma unroll
+    for (int m = 0; m < L; ++m) F[m + 1] = F[m] * (m + 0.5) * it;
+}
 
 // tab: the aligned per-L tables (see BOYS_LA).
 template <int L>
@@ -139,65 +187,25 @@ POLY_HD void boys_fp64(double T, double pref, const double* __restrict__ tab,
     static_assert(L < BOYS_LA, "Boys table too short for this class");
     if (T < BOYS_TMAX) {
         const int ts = (int)(T * 20.0 + 0.5);
-        const double h = 0.05 * ts - T;
-        const BoysPair* g = reinterpret_cast<const BoysPair*>(tab + ((size_t)L * BOYS_NT + ts) * 8);
-        const BoysPair g01 = g[0], g23 = g[1], g45 = g[2];
-        double f = tab[((size_t)L * BOYS_NT + ts) * 8 + 6];
-        f = g45.y + h * (1.0 / 6.0) * f;
-        f = g45.x + h * (1.0 / 5.0) * f;
-        f = g23.y + h * (1.0 / 4.0) * f;
-        f = g23.x + h * (1.0 / 3.0) * f;
-        f = g01.y + h * (1.0 / 2.0) * f;
-        f = g01.x + h * f;
-        F[L] = f;
-        if (L > 0) {
-            const double e = exp(-T);
-            const double t2 = 2.0 * T;
-#pragma unroll
-            for (int m = L - 1; m >= 0; --m) F[m] = (t2 * F[m + 1] + e) * (1.0 / (2 * m + 1));
-        }
+        boys_rows<L, 8>(T, 0.05 * ts - T, tab + ((size_t)L * BOYS_NT + ts) * 8, F);
     } else {
-        const double r = rsqrt_fp64(T), it = r * r;
-        F[0] = 0.5 * POLY_SQRT_PI * r;
-#pragma unroll
-        for (int m = 0; m < L; ++m) F[m + 1] = F[m] * (m + 0.5) * it;
+        boys_large<L>(T, F);
     }
 #pragma unroll
     for (int m = 0; m <= L; ++m) F[m] *= pref;
 }
 
 // The same from the coarse rows of one L (row0: BOYS_CNT rows of ten
-// values, in LDS), same downward recursion and asymptotic form.
+// coefficients, in LDS).
 template <int L>
 POLY_HD void boys_coarse(double T, double pref, const double* __restrict__ row0, double* __restrict__ F) {
     static_assert(L < BOYS_LC, "coarse Boys table too short for this class");
     if (T < BOYS_TMAX) {
-        const int ts = (int)(T * 5.0 + 0.5);
-        const double h = 0.2 * ts - T;
-        const BoysPair* g = reinterpret_cast<const BoysPair*>(row0 + ts * 10);
-        const BoysPair g01 = g[0], g23 = g[1], g45 = g[2], g67 = g[3], g89 = g[4];
-        double f = g89.y;
-        f = g89.x + h * (1.0 / 9.0) * f;
-        f = g67.y + h * (1.0 / 8.0) * f;
-        f = g67.x + h * (1.0 / 7.0) * f;
-        f = g45.y + h * (1.0 / 6.0) * f;
-        f = g45.x + h * (1.0 / 5.0) * f;
-        f = g23.y + h * (1.0 / 4.0) * f;
-        f = g23.x + h * (1.0 / 3.0) * f;
-        f = g01.y + h * (1.0 / 2.0) * f;
-        f = g01.x + h * f;
-        F[L] = f;
-        if (L > 0) {
-            const double e = exp(-T);
-            const double t2 = 2.0 * T;
-#pragma unroll
-            for (int m = L - 1; m >= 0; --m) F[m] = (t2 * F[m + 1] + e) * (1.0 / (2 * m + 1));
-        }
+        int ts = (int)(T * (20.0 / 3.0) + 0.5);
+        if (ts > BOYS_CNT - 1) ts = BOYS_CNT - 1;
+        boys_rows<L, 10>(T, 0.15 * ts - T, row0 + ts * 10, F);
     } else {
-        const double r = rsqrt_fp64(T), it = r * r;
-        F[0] = 0.5 * POLY_SQRT_PI * r;
-#pragma unroll
-        for (int m = 0; m < L; ++m) F[m + 1] = F[m] * (m + 0.5) * it;
+        boys_large<L>(T, F);
     }
 #pragma unroll
     for (int m = 0; m <= L; ++m) F[m] *= pref;
@@ -271,7 +279,7 @@ POLY_HD void prim_vrr(const PrimPair& bp, const PrimPair& kq, const double* __re
     ClassCode<LA, LB, LC, LD, real>::vrr(
         (real)bp.PAx, (real)bp.PAy, (real)bp.PAz, (real)(-roz * PQx), (real)(-roz * PQy), (real)(-roz * PQz),
         (real)kq.PAx, (real)kq.PAy, (real)kq.PAz, (real)(roe * PQx), (real)(roe * PQy), (real)(roe * PQz),
-        (real)(0.5 / bp.zeta), (real)(0.5 / kq.zeta), (real)(0.5 * ize), (real)roz, (real)roe, Fr, acc);
+        (real)bp.h, (real)kq.h, (real)(0.5 * ize), (real)roz, (real)roe, Fr, acc);
 }
 
 // Contracted (ab|cd) for one shell quartet.  bra/ket point at the

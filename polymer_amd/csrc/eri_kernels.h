@@ -57,7 +57,7 @@ struct EriArgs {
     int tpack;                 // MODE_TENSOR: the pair-packed layout of TensorCb
     const int2* items;         // explicit (bra pair, ket position) items of a density-screened list, or null
     const unsigned* count;     // number of items (device), with items
-    const double* ksoa;        // ket primitive pairs, bucket-interleaved fields (8 x kfs doubles)
+    const double* ksoa;        // ket primitive pairs, bucket-interleaved fields (9 x kfs doubles)
     long long kfs;             // field stride of ksoa
     const int* bucket_soa;     // nbucket: offset of each ket bucket in ksoa
     // periodic (MODE_PBC): nwork = items x n3, Q3 = t % n3 - cel2
@@ -702,6 +702,31 @@ __global__ void __launch_bounds__(256) k_eri(EriArgs g) {
         eri_item<LA, LB, LC, LD, MODE>(g, t);
 }
 
+// Primitive pairs at an address that is the same for the whole wavefront,
+// through the scalar cache.  In a loop with J/K atomics the compiler takes a
+// plain load of them for a vector one (the atomics might write there): in
+// k_eri_gc that was 26 registers and eleven loads a primitive quartet, each
+// returning the same words to 64 lanes.
+typedef const __attribute__((address_space(4))) double* ScalarDoubles;
+__device__ __forceinline__ PrimPair scalar_pair(ScalarDoubles x) {
+    PrimPair r;
+    r.zeta = x[0]; r.K = x[1]; r.Px = x[2]; r.Py = x[3]; r.Pz = x[4];
+    r.PAx = x[5]; r.PAy = x[6]; r.PAz = x[7]; r.h = x[8];
+    return r;
+}
+__device__ __forceinline__ PrimPair scalar_load(const PrimPair* p) {
+    static_assert(sizeof(PrimPair) == 9 * sizeof(double), "field order of scalar_pair");
+    return scalar_pair((ScalarDoubles)p);
+}
+__device__ __forceinline__ GcPrim scalar_load(const GcPrim* p) {
+    static_assert(sizeof(GcPrim) == 13 * sizeof(double), "field order");
+    const ScalarDoubles x = (ScalarDoubles)p;
+    GcPrim r;
+    r.pp = scalar_pair(x);
+    for (int i = 0; i < 4; ++i) r.w[i] = x[9 + i];
+    return r;
+}
+
 // Sums over the lanes that share one item.  The 2^ls lanes of an item are
 // those that differ in lane bits 5, 4, .. 6 - ls, so step S of a reduction
 // exchanges with the lane whose bit 5 - S differs, whatever ls is.
@@ -796,14 +821,24 @@ __device__ __forceinline__ double wave_sum(double v) {
 }
 
 // SHARE: the form for lists in which some segments share items between
-// lanes; without it every item has one lane.
-template <int LA, int LB, int LC, int LD, int MODE, bool SHARE>
+// lanes; without it every item has one lane.  BT: the block copies the
+// coarse Boys rows of its L into LDS, in front of the rows, and reads them
+// there.
+template <int LA, int LB, int LC, int LD, int MODE, bool SHARE, bool BT>
 __global__ void __launch_bounds__(256) k_eri_seg(EriArgs g) {
     constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
     constexpr int NE = ((LA + LB + 1) * (LA + LB + 2) * (LA + LB + 3) - LA * (LA + 1) * (LA + 2)) / 6;
     constexpr int NF = ((LC + LD + 1) * (LC + LD + 2) * (LC + LD + 3) - LC * (LC + 1) * (LC + 2)) / 6;
     using real = typename std::conditional<MODE == MODE_JK32, float, double>::type;
-    extern __shared__ double seg_lds[];
+    extern __shared__ double lds_all[];
+    const double* btab = g.boysA;
+    double* seg_lds = lds_all;
+    if (BT) {
+        const double* src = g.boys + BOYS_COFF + (size_t)(LA + LB + LC + LD) * BOYS_CROWS;
+        for (int i = threadIdx.x; i < BOYS_CROWS; i += blockDim.x) lds_all[i] = src[i];
+        btab = lds_all;
+        seg_lds = lds_all + BOYS_CROWS;      // the first zeroing pass below is followed by a barrier
+    }
     const int n = g.nbf;
     double* Kr = seg_lds;                        // rows fa.. (NA) then fb.. (NB), width n
     double* Jl = seg_lds + (size_t)(NA + NB) * n;
@@ -854,10 +889,12 @@ __global__ void __launch_bounds__(256) k_eri_seg(EriArgs g) {
             real acc[NE * NF];
 #pragma unroll
             for (int i = 0; i < NE * NF; ++i) acc[i] = real(0);
-            for (int p = 0; p < mb.nprim; ++p) {
-                const PrimPair bq = bra[p];
-                for (int q = sub; q < nkp; q += 1 << ls)
-                    prim_vrr<real, LA, LB, LC, LD>(bq, kv.load(q), g.boysA, acc);
+            // ket primitive outer (its fields stay in registers), bra inner
+            // (the same for the whole block: scalar loads)
+            for (int q = sub; q < nkp; q += 1 << ls) {
+                const PrimPair kq = kv.load(q);
+                for (int p = 0; p < mb.nprim; ++p)
+                    prim_vrr<real, LA, LB, LC, LD, BT>(scalar_load(bra + p), kq, btab, acc);
             }
             if constexpr (SHARE) {
                 if (ls) {
@@ -970,9 +1007,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LA + L
 k_eri_gc(EriArgs g) {
     constexpr int NA = ncart(LA), NC = ncart(LC), NI = NA * NC;
     constexpr int MB = LA == 0 ? 4 : 2, MK = LC == 0 ? 4 : 2;
-    // factored member weights for (ss|ss) (measured faster there, no change
-    // for the other classes, whose bra sums cost registers)
-    constexpr bool GC_FACTOR = LA == 0 && LC == 0;
     extern __shared__ double lds_all[];
     const double* btab = g.boysA;
     double* seg_lds = lds_all;
@@ -1042,54 +1076,30 @@ k_eri_gc(EriArgs g) {
                 PrimPair kq;
                 kq.zeta = x[0]; kq.K = x[fs]; kq.Px = x[2 * fs]; kq.Py = x[3 * fs]; kq.Pz = x[4 * fs];
                 kq.PAx = x[5 * fs]; kq.PAy = x[6 * fs]; kq.PAz = x[7 * fs];
-                if (GC_FACTOR) {
-                    // sum over the bra primitives with the bra members'
-                    // weights, then apply the ket members' weights once per
-                    // ket primitive
-                    double sb[MB * NI];
+                kq.h = 0.0;                     // kets (s s| and (p s| do not enter it
+                // sum over the bra primitives with the bra members' weights,
+                // then apply the ket members' weights once per ket primitive
+                double sb[MB * NI];
 #pragma unroll
-                    for (int i = 0; i < MB * NI; ++i) sb[i] = 0.0;
-                    for (int p = 0; p < mb.nprim; ++p) {
-                        const GcPrim bq = bra[p];
-                        double tv[NI];
+                for (int i = 0; i < MB * NI; ++i) sb[i] = 0.0;
+                for (int p = 0; p < mb.nprim; ++p) {
+                    const GcPrim bq = scalar_load(bra + p);
+                    double tv[NI];
 #pragma unroll
-                        for (int i = 0; i < NI; ++i) tv[i] = 0.0;
-                        prim_vrr<double, LA, 0, LC, 0, BT>(bq.pp, kq, btab, tv);
+                    for (int i = 0; i < NI; ++i) tv[i] = 0.0;
+                    prim_vrr<double, LA, 0, LC, 0, BT>(bq.pp, kq, btab, tv);
 #pragma unroll
-                        for (int i = 0; i < MB; ++i)
+                    for (int i = 0; i < MB; ++i)
 #pragma unroll
-                            for (int e = 0; e < NI; ++e) sb[i * NI + e] += bq.w[i] * tv[e];
-                    }
+                        for (int e = 0; e < NI; ++e) sb[i * NI + e] += bq.w[i] * tv[e];
+                }
 #pragma unroll
-                    for (int j = 0; j < MK; ++j) {
-                        const double wk = x[(8 + j) * fs];
+                for (int j = 0; j < MK; ++j) {
+                    const double wk = x[(8 + j) * fs];
 #pragma unroll
-                        for (int i = 0; i < MB; ++i)
+                    for (int i = 0; i < MB; ++i)
 #pragma unroll
-                            for (int e = 0; e < NI; ++e) acc[(i * MK + j) * NI + e] += wk * sb[i * NI + e];
-                    }
-                } else {
-                    double wk[MK];
-#pragma unroll
-                    for (int j = 0; j < MK; ++j) wk[j] = x[(8 + j) * fs];
-                    for (int p = 0; p < mb.nprim; ++p) {
-                        const GcPrim bq = bra[p];
-                        double tv[NI];
-#pragma unroll
-                        for (int i = 0; i < NI; ++i) tv[i] = 0.0;
-                        prim_vrr<double, LA, 0, LC, 0, BT>(bq.pp, kq, btab, tv);
-                        double u[MB * NI];
-#pragma unroll
-                        for (int i = 0; i < MB; ++i)
-#pragma unroll
-                            for (int e = 0; e < NI; ++e) u[i * NI + e] = bq.w[i] * tv[e];
-#pragma unroll
-                        for (int j = 0; j < MK; ++j)
-#pragma unroll
-                            for (int i = 0; i < MB; ++i)
-#pragma unroll
-                                for (int e = 0; e < NI; ++e) acc[(i * MK + j) * NI + e] += wk[j] * u[i * NI + e];
-                    }
+                        for (int e = 0; e < NI; ++e) acc[(i * MK + j) * NI + e] += wk * sb[i * NI + e];
                 }
             }
             int i0 = 0, ni = MB, j0 = 0, nj = MK;
@@ -1331,10 +1341,11 @@ __global__ void __launch_bounds__(256) k_eri_gck(EriArgs g) {
                 PrimPair kq;
                 kq.zeta = x[0]; kq.K = x[fs]; kq.Px = x[2 * fs]; kq.Py = x[3 * fs]; kq.Pz = x[4 * fs];
                 kq.PAx = x[5 * fs]; kq.PAy = x[6 * fs]; kq.PAz = x[7 * fs];
+                kq.h = 0.0;                     // kets (s s| and (p s| do not enter it
                 double sb[NE * NF];
 #pragma unroll
                 for (int i = 0; i < NE * NF; ++i) sb[i] = 0.0;
-                for (int p = 0; p < mb.nprim; ++p) prim_vrr<double, LA, LB, LC, 0, BT>(bra[p], kq, btab, sb);
+                for (int p = 0; p < mb.nprim; ++p) prim_vrr<double, LA, LB, LC, 0, BT>(scalar_load(bra + p), kq, btab, sb);
 #pragma unroll
                 for (int j = 0; j < MK; ++j) {
                     const double wk = x[(8 + j) * fs];
@@ -1400,8 +1411,9 @@ __global__ void __launch_bounds__(256) k_eri_gck(EriArgs g) {
 typedef void (*EriKernel)(EriArgs);
 // Getter modes of polyeri_class_kernel beyond the k_eri modes: the segment
 // kernel for MODE_JK and MODE_JK32, and for MODE_JK with items shared between
-// lanes.
-enum { GET_SEG_JK = 5, GET_SEG_JK32 = 6, GET_SEG_SHARE = 7 };
+// lanes; GET_SEG_SHARE_G is the last with the Boys rows read from global memory
+// (GET_SEG_JK and GET_SEG_SHARE need BOYS_CROWS doubles more LDS).
+enum { GET_SEG_JK = 5, GET_SEG_JK32 = 6, GET_SEG_SHARE = 7, GET_SEG_SHARE_G = 8 };
 // Strided batched FP64 products on the MFMA units (kgemm.hip):
 // C_b(m,n) = sum_k A_b(m,k) B_b(k,n), X_b(r,c) = X[b*sX + r*sXr + c*sXc].
 enum { GEMM_F64 = 1, GEMM_BF16X3 = 2 };

@@ -256,10 +256,9 @@ def write_kernel_units(out_dir):
             body.append("    switch (mode) {")
             for m in range(5):
                 body.append(f"    case {m}: return k_eri<{la}, {lb}, {lc}, {ld}, {m}>;")
-            # getter modes 5 and 6: the segment kernel in FP64 and mixed precision
-            body.append(f"    case 5: return k_eri_seg<{la}, {lb}, {lc}, {ld}, 0, false>;")
-            body.append(f"    case 6: return k_eri_seg<{la}, {lb}, {lc}, {ld}, 3, false>;")
-            body.append(f"    case 7: return k_eri_seg<{la}, {lb}, {lc}, {ld}, 0, true>;")
+            # getter modes 5 .. 8: the forms of the segment kernel
+            for m, form in ((5, "0, false, true"), (6, "3, false, false"), (7, "0, true, true"), (8, "0, true, false")):
+                body.append(f"    case {m}: return k_eri_seg<{la}, {lb}, {lc}, {ld}, {form}>;")
             body += ["    }", "    return nullptr;", "}", ""]
         text = "\n".join(body)
         if not os.path.exists(path) or open(path).read() != text:

@@ -152,7 +152,7 @@ __device__ __forceinline__ void rys_variant(const EriArgs& g, const SegDesc& seg
 #pragma unroll
         for (int i = 0; i < R::NOUT; ++i) accr[i] = real(0);
         for (int pi = 0; pi < nbra; ++pi) {
-            const PrimPair bq = bra[pi];
+            const PrimPair bq = scalar_load(bra + pi);
             const double PAg[3] = {bq.PAx, bq.PAy, bq.PAz};
             const double PA0 = sel3(PAg, p[0]), PA1 = sel3(PAg, p[1]), PA2 = sel3(PAg, p[2]);
             for (int qi = 0; qi < mk.nprim; ++qi)
@@ -401,6 +401,7 @@ static void rys_block_host_var(const PrimPair& bq, const PrimPair& kq, const dou
 static PrimPair host_prim_pair(double a, const double* A, double b, const double* B) {
     PrimPair q;
     q.zeta = a + b;
+    q.h = 0.5 / q.zeta;
     const double d2 = (A[0] - B[0]) * (A[0] - B[0]) + (A[1] - B[1]) * (A[1] - B[1]) + (A[2] - B[2]) * (A[2] - B[2]);
     q.K = std::sqrt(2.0) * std::pow(3.141592653589793, 1.25) * std::exp(-a * b / q.zeta * d2) / q.zeta;
     q.Px = (a * A[0] + b * B[0]) / q.zeta;

@@ -690,8 +690,15 @@ static int launch_class(polyeri_ctx* c, int mode, int la, int lb, int lc, int ld
         }
     }
     if (kind == LAUNCH_SEG) {
-        EriKernel ks = polyeri_class_kernel(
-            la, lb, lc, ld, mode != MODE_JK ? GET_SEG_JK32 : share ? GET_SEG_SHARE : GET_SEG_JK);
+        // the coarse Boys rows go into LDS where they fit beside the rows
+        size_t lds = seg_lds_bytes(la, lb, c->ib.nbf);
+        const bool bt = mode == MODE_JK && lds + BOYS_CROWS * sizeof(double) <= 65536;
+        if (bt) lds += BOYS_CROWS * sizeof(double);
+        EriKernel ks = polyeri_class_kernel(la, lb, lc, ld,
+                                            mode != MODE_JK ? GET_SEG_JK32
+                                            : !bt           ? GET_SEG_SHARE_G
+                                            : share         ? GET_SEG_SHARE
+                                                            : GET_SEG_JK);
         if (!ks) return fail(POLYERI_E_ARG, "no segment kernel for class");
         a.segs = segs;
         a.nseg = nseg;
@@ -702,7 +709,7 @@ static int launch_class(polyeri_ctx* c, int mode, int la, int lb, int lc, int ld
         const int block = cfg.block == 64 || cfg.block == 128 ? cfg.block : 256;
         unsigned grid = (unsigned)nseg;
         if (cfg.grid > 0 && grid > (unsigned)cfg.grid) grid = (unsigned)cfg.grid;
-        hipLaunchKernelGGL(ks, dim3(grid), dim3(block), seg_lds_bytes(la, lb, c->ib.nbf), c->stream, a);
+        hipLaunchKernelGGL(ks, dim3(grid), dim3(block), lds, c->stream, a);
         HIPCHK(hipGetLastError());
         return 0;
     }
@@ -1127,21 +1134,25 @@ static int build_ctx(polyeri_ctx* c) {
     if ((rc = dalloc(&c->d_prims, c->prims.size()))) return rc;
     if ((rc = dalloc(&c->d_meta, np))) return rc;
     if ((rc = dalloc(&c->d_ab, 4 * (size_t)np))) return rc;
-    // device copy: the BOYS_NT x BOYS_NM table, then the aligned per-L tables
-    // of the thread kernels (BOYS_LA x BOYS_NT rows of F_L .. F_{L+6}, pad),
-    // then the coarse per-L rows (BOYS_LC x BOYS_CNT rows of F_L .. F_{L+9}
-    // at every fourth grid point)
-    static_assert(BOYS_LC - 1 + 9 < BOYS_NM && 4 * (BOYS_CNT - 1) < BOYS_NT, "coarse Boys rows out of the table");
+    // device copy: the BOYS_NT x BOYS_NM table, then the aligned per-L rows
+    // of the thread kernels, then the coarse per-L rows (eri_engine.h)
+    static_assert(BOYS_LC - 2 + 9 < BOYS_NM && BOYS_LA - 2 + 7 < BOYS_NM && 3 * (BOYS_CNT - 1) < BOYS_NT,
+                  "Boys rows out of the table");
     std::vector<double> boys_dev(boys);
     boys_dev.resize((size_t)BOYS_COFF + (size_t)BOYS_LC * BOYS_CROWS, 0.0);
+    auto row = [&](double* out, int n, int L, int i) {
+        const double* f = boys.data() + (size_t)i * BOYS_NM + (L > 0 ? L - 1 : 0);
+        double fact = 1.0;
+        for (int k = 0; k < n; ++k) {
+            out[k] = f[k] / fact;
+            fact *= k + 1;
+        }
+    };
     for (int L = 0; L < BOYS_LA; ++L)
-        for (int i = 0; i < BOYS_NT; ++i)
-            for (int j = 0; j < 7; ++j)
-                boys_dev[(size_t)BOYS_AOFF + ((size_t)L * BOYS_NT + i) * 8 + j] = boys[(size_t)i * BOYS_NM + L + j];
+        for (int i = 0; i < BOYS_NT; ++i) row(boys_dev.data() + BOYS_AOFF + ((size_t)L * BOYS_NT + i) * 8, 8, L, i);
     for (int L = 0; L < BOYS_LC; ++L)
-        for (int i = 0; i < BOYS_CNT; ++i)
-            for (int j = 0; j < 10; ++j)
-                boys_dev[(size_t)BOYS_COFF + (size_t)L * BOYS_CROWS + i * 10 + j] = boys[(size_t)4 * i * BOYS_NM + L + j];
+        for (int j = 0; j < BOYS_CNT; ++j)
+            row(boys_dev.data() + BOYS_COFF + (size_t)L * BOYS_CROWS + j * 10, 10, L, 3 * j);
     if ((rc = dalloc(&c->d_boys, boys_dev.size()))) return rc;
     if ((rc = dalloc(&c->d_Q, np))) return rc;
     if ((rc = dalloc(&c->d_ref, nbf))) return rc;
@@ -1215,7 +1226,7 @@ static int build_ctx(polyeri_ctx* c) {
     }
     {
         const size_t P = c->prims.size();
-        std::vector<double> soa(8 * P, 0.0);
+        std::vector<double> soa(9 * P, 0.0);
         size_t off = 0;
         for (int Y = 0; Y < NPAIRCLASS; ++Y) {
             const auto& kl = c->ket_ids[Y];
@@ -1230,8 +1241,8 @@ static int build_ctx(polyeri_ctx* c) {
                     for (int q = 0; q < np_b; ++q) {
                         const PrimPair& pp = c->prims[pi.prim_off + q];
                         const size_t at = off + (size_t)q * nk + i;
-                        const double f[8] = {pp.zeta, pp.K, pp.Px, pp.Py, pp.Pz, pp.PAx, pp.PAy, pp.PAz};
-                        for (int k = 0; k < 8; ++k) soa[k * P + at] = f[k];
+                        const double f[9] = {pp.zeta, pp.K, pp.Px, pp.Py, pp.Pz, pp.PAx, pp.PAy, pp.PAz, pp.h};
+                        for (int k = 0; k < 9; ++k) soa[k * P + at] = f[k];
                     }
                 }
                 off += (size_t)np_b * nk;
