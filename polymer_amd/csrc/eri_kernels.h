@@ -706,7 +706,7 @@ __global__ void __launch_bounds__(256) k_eri(EriArgs g) {
 // through the scalar cache.  In a loop with J/K atomics the compiler takes a
 // plain load of them for a vector one (the atomics might write there): in
 // k_eri_gc that was 26 registers and eleven loads a primitive quartet, each
-// returning the same words to 64 lanes.
+// returning the same words to 64 lanes ((ps|ss) of (H2O)16 2.56 -> 2.21 ms).
 typedef const __attribute__((address_space(4))) double* ScalarDoubles;
 __device__ __forceinline__ PrimPair scalar_pair(ScalarDoubles x) {
     PrimPair r;
@@ -814,6 +814,11 @@ __device__ __forceinline__ void lane_reduce(double* acc, int ls, int lane, int& 
 // registers (J_ab, reduced over the wavefront), and added to the XCD's J/K
 // copy once per segment, one atomic per nonzero element.  Only J_cd is added
 // per quartet.  LDS: ((NA + NB) nbf + NA NB) doubles.
+// Bound by the loads and atomics of the digestion (texture data path 60-75 %
+// busy, FP64 VALU 25-60 %).  With the ket primitive outside, the bra's in
+// scalar registers and the Boys rows in LDS no vector load is left in the
+// inner loop: C16H34 6-31G** (ss|ss) 0.69 -> 0.44, (ps|ss) 1.18 -> 0.89 ms,
+// (H2O)16 cc-pVDZ (pp|ss) 1.38 -> 0.95, (pp|ps) 1.63 -> 1.49 ms.
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -964,7 +969,9 @@ __global__ void __launch_bounds__(256) k_eri_seg(EriArgs g) {
     }
 }
 
-// Segment kernel of the generally contracted lists, classes (ls|l's): as
+// Segment kernel of the generally contracted lists, classes (ls|l's)
+// ((H2O)16: (ss|ss) 2.9 -> 1.2 ms with shared items and scalar bra loads,
+// (ps|ss) 3.1 -> 2.2, (ps|ps) 2.6 -> 1.9; FP64 VALU 38-53 % busy): as
 // k_eri_seg, but an item is a pair of generally contracted pairs (GcMeta)
 // and computes all member quartets from one primitive loop: for each ket
 // primitive, the primitive quartets' [a0|c0] blocks are summed over the bra

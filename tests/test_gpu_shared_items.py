@@ -9,6 +9,7 @@ import pytest
 
 import oracle
 import polymer_amd as pa
+from polymer_amd import geometry
 from tests.conftest import basis_path
 from tests.molecules import BH_GOLDEN, H2O_GOLDEN
 
@@ -47,3 +48,33 @@ def test_shared_items_match_oracle(case, grouped):
     js, ks = ctx.fourindex_eri(p, dens_tol=1e-290)
     assert np.max(np.abs(js - jr)) < 1e-10 and np.max(np.abs(ks - kr)) < 1e-10
     assert ctx.stats()["last_quartets"] >= n       # every quartet kept
+
+
+def test_boys_rows_outside_lds_match_register_kernels():
+    """Above about 450 functions the (dd|..) rows leave no LDS for the Boys
+    rows and the segment kernel reads them from global memory; both it and
+    the LDS form of the other classes against the thread-per-quartet kernels
+    on the same quartets.  Tolerance: 10^6 terms of at most 1 a matrix
+    element, 10^6 x 2^-53 = 1.2e-10, doubled for the two orders of summation."""
+    atoms = geometry.water_cluster(19, 2, radius=5.5)
+    print("case: Boys rows from global memory, (H2O)19 cc-pVDZ", flush=True)
+    b = pa.read_basis("cc-pVDZ", atoms)
+    ctx = pa.Context(b, schwarz_tol=1e-9)
+    ctx.set_general_contraction(False)
+    rng = np.random.default_rng(3)
+    real = b.real_functions
+    p = np.zeros((b.ncgs, b.ncgs))
+    a = 0.05 * rng.standard_normal((len(real), 12))
+    p[np.ix_(real, real)] = a @ a.T
+    j, k = ctx.fourindex_eri(p)
+    cls = ctx.stats()["classes"]
+    kinds = {c["cls"]: c["kernel"] for c in cls if c["quartets"]}
+    assert kinds["2200"] == "seg" and kinds["0000"] == "seg", kinds
+    cfg = ctx.launch_configs()
+    for c, x in zip(cfg, cls):
+        if x["kernel"] == "seg":
+            c[0], c[1], c[2] = 1, 256, 0
+    ctx.set_launch_configs(cfg)
+    jr, kr = ctx.fourindex_eri(p)
+    assert np.max(np.abs(jr)) > 1
+    assert np.max(np.abs(j - jr)) < 2.4e-10 and np.max(np.abs(k - kr)) < 2.4e-10
