@@ -52,6 +52,7 @@ struct PrimPair {
     double Px, Py, Pz;
     double PAx, PAy, PAz;
     double h;   // 1 / (2 zeta): stored, a division costs ten FP64 instructions a primitive quartet
+    double a2;  // twice the first shell's exponent (gradient)
 };
 
 // Generally contracted pair (classes (ls|), s shells that share exponents):

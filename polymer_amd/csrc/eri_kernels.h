@@ -711,19 +711,19 @@ typedef const __attribute__((address_space(4))) double* ScalarDoubles;
 __device__ __forceinline__ PrimPair scalar_pair(ScalarDoubles x) {
     PrimPair r;
     r.zeta = x[0]; r.K = x[1]; r.Px = x[2]; r.Py = x[3]; r.Pz = x[4];
-    r.PAx = x[5]; r.PAy = x[6]; r.PAz = x[7]; r.h = x[8];
+    r.PAx = x[5]; r.PAy = x[6]; r.PAz = x[7]; r.h = x[8]; r.a2 = x[9];
     return r;
 }
 __device__ __forceinline__ PrimPair scalar_load(const PrimPair* p) {
-    static_assert(sizeof(PrimPair) == 9 * sizeof(double), "field order of scalar_pair");
+    static_assert(sizeof(PrimPair) == 10 * sizeof(double), "field order of scalar_pair");
     return scalar_pair((ScalarDoubles)p);
 }
 __device__ __forceinline__ GcPrim scalar_load(const GcPrim* p) {
-    static_assert(sizeof(GcPrim) == 13 * sizeof(double), "field order");
+    static_assert(sizeof(GcPrim) == 14 * sizeof(double), "field order");
     const ScalarDoubles x = (ScalarDoubles)p;
     GcPrim r;
     r.pp = scalar_pair(x);
-    for (int i = 0; i < 4; ++i) r.w[i] = x[9 + i];
+    for (int i = 0; i < 4; ++i) r.w[i] = x[10 + i];
     return r;
 }
 
@@ -1476,63 +1476,75 @@ int polyeri_rys_nodes_host(int n, double T, double* u, double* w);
 // exactly once).
 int polyeri_rys_block_host(int la, int lb, int lc, int ld, const double* xyz, const double* ex, double* out);
 
-// Two-electron part of the nuclear gradient (kgrad.hip): shells of the
-// library's basis (L, atom, first function, first primitive, primitive
-// count, centre), primitive exponents and coefficients, the density in the
-// library's basis (nbf x nbf) and its largest |element| per shell block
-// (nsh x nsh), the per-pair Schwarz bounds (filled by the launcher), the
-// threshold on Q_ab Q_cd and on Q_ab Q_cd max |Gamma|, the exchange scale.
-// Shell pairs (pa[i], pb[i]) with L(pa) >= L(pb), grouped by pair class
+// Two-electron part of the nuclear gradient (kgrad.hip): per shell its atom,
+// first function and centre, the density in the library's basis (nbf x nbf)
+// and its largest |element| per shell block (nsh x nsh), the threshold on
+// Q_ab Q_cd and on Q_ab Q_cd max |Gamma|, the exchange scale.
+// Shell pairs (pa[i], pb[i]) with L(pa) >= L(pb), their Schwarz bounds and
+// their primitive pairs prims[pp0[i]] .. + pn[i] - 1, grouped by pair class
 // ((ss) (ps) (pp) (ds) (dp) (dd) = 0 .. 5: pairs seg[X] .. seg[X + 1] - 1),
 // by primitive count inside a class; the quartets of class pair X >= Y run
 // as one launch of the kernel for that class.
 struct GradArgs {
     int nsh, natom, nbf, npair;
     int seg[7];
-    const int *L, *atom, *f0, *p0, *np;
-    const int *pa, *pb;
-    const double *xyz, *alpha, *coef;
+    const int *atom, *f0;
+    const int *pa, *pb, *pp0, *pn;
+    const PrimPair* prims;
+    const double* xyz;
     const double* D;
     const double* dsh;
     const double* Qp;
-    double tol, xfac, ptol;
-    // the Schwarz survivors of one class pair as chunks: chunk c holds the
-    // quartets coff[c] .. coff[c + 1] - 1, bra pair x0 + cij[2c] and ket
-    // pairs y0 + cij[2c + 1] + (t - coff[c]); null: the full product
+    double tol, xfac;
+    // the Schwarz survivors of one class pair as chunks: chunk c holds lanes
+    // coff[c] .. coff[c + 1] - 1, cij[3c + 2] to a quartet of bra pair x0 +
+    // cij[3c] and ket pairs y0 + cij[3c + 1] + 0, 1, ..
     const unsigned long long* coff = nullptr;
     const int* cij = nullptr;
     int nchunk = 0;
 };
+// One root of a primitive quartet is a unit of work in the classes of this
+// many integrals and more, a whole primitive quartet below.
+constexpr bool grad_root_units(int nint) { return nint >= 36; }
+
+// Shells and primitives for the host's Schwarz bounds, ptol the primitive
+// pair threshold.
+struct GradShells {
+    const int *L, *p0, *np;
+    const double *xyz, *alpha, *coef;
+    double ptol;
+};
 
 // Schwarz-surviving quartets of every class pair (X, Y <= X) of pairs sorted
 // by polyeri_grad_sort_pairs: inside a class, pairs of one primitive count
-// (a group) are in descending bound order, so the kets of a group that
+// class (a group) are in descending bound order, so the kets of a group that
 // survive with a given bra are a prefix of the group.  Class pair k = 6X + Y
-// has n[k] chunks, offsets off[off0[k]] .. off[off0[k] + n[k]] and
-// (row, first column) pairs ij[ij0[k] ..].
+// has n[k] chunks, offsets off[off0[k]] .. off[off0[k] + n[k]] (in lanes) and
+// (row, first column, lanes a quartet) triples ij[ij0[k] ..].
 struct GradChunks {
     std::vector<unsigned long long> off;
     std::vector<int> ij;
     size_t off0[36], ij0[36];
     int n[36];
-    unsigned long long nq[36];
+    unsigned long long nlane[36];
+    double units[36];
 };
-// grad (3 natom, zeroed by the caller) += dE2/dR on the device; d_Qp: npair
-// doubles, the pair bounds when have_qp, else computed here.  ch (optional,
-// with d_off / d_ij its off / ij arrays on the device): launch only the
-// Schwarz survivors it lists.
-int polyeri_grad_launch(const GradArgs& g, double* d_Qp, double* d_grad, hipStream_t stream, bool have_qp = false,
-                        const GradChunks* ch = nullptr, const unsigned long long* d_off = nullptr,
-                        const int* d_ij = nullptr);
-// Orders the pairs of every class segment by primitive count (descending,
-// as they come) and, inside one count, by bound (descending); pa, pb and qp
+// grad (3 natom, zeroed by the caller) += dE2/dR on the device: the chunks ch
+// (with d_off / d_ij its off / ij arrays on the device), the class pairs dealt
+// over the ns streams, costliest first.
+int polyeri_grad_launch(const GradArgs& g, double* d_grad, const hipStream_t* streams, int ns, const GradChunks& ch,
+                        const unsigned long long* d_off, const int* d_ij);
+// Orders the pairs of every class segment by primitive count class
+// (descending) and, inside one, by bound (descending); pa, pb, qp, pp0 and pn
 // permuted together.  False (nothing changed) when a bound is not finite.
-bool polyeri_grad_sort_pairs(int* pa, int* pb, double* qp, const int* np, const int* seg);
-// The chunks of sorted pairs whose bound product is >= tol.
-void polyeri_grad_chunks(const int* pa, const int* pb, const int* np, const double* qp, const int* seg, double tol,
+bool polyeri_grad_sort_pairs(int* pa, int* pb, double* qp, int* pp0, int* pn, const int* seg);
+// The chunks of the pairs whose bound product is >= tol (sorted = false: of
+// all pairs, in their order); split: several lanes to a quartet.
+void polyeri_grad_chunks(const double* qp, const int* pn, const int* seg, double tol, bool sorted, bool split,
                          GradChunks& ch);
-// the same sum on the host (host pointers), grad overwritten
-int polyeri_grad_host(const GradArgs& g, double* grad);
+// the same sum on the host (host pointers), grad overwritten, Schwarz bounds
+// from gs
+int polyeri_grad_host(const GradArgs& g, const GradShells& gs, double* grad);
 // One record of the reference's .ao files (kstored.hip): packed cells,
 // packed 1-based indices I J K L, the integral.
 struct StoredEri {

@@ -324,6 +324,7 @@ void build_pairs(const IntBasis& ib, double primtol, std::vector<PairInfo>& pair
                     PrimPair pp;
                     pp.zeta = z;
                     pp.h = 0.5 / z;
+                    pp.a2 = 2.0 * al;
                     pp.K = cc * e * c0 / z;
                     pp.Px = (al * A.x + be * B.x) / z;
                     pp.Py = (al * A.y + be * B.y) / z;
@@ -413,6 +414,7 @@ int build_gc_pairs(const IntBasis& ib, double primtol, const std::vector<PairInf
                     if (wmax * e < primtol) continue;
                     gp.pp.zeta = z;
                     gp.pp.h = 0.5 / gp.pp.zeta;
+                    gp.pp.a2 = 2.0 * al;
                     gp.pp.K = e * c0 / z;
                     gp.pp.Px = (al * A.x + be * B.x) / z;
                     gp.pp.Py = (al * A.y + be * B.y) / z;
@@ -471,6 +473,7 @@ void build_pairs_cells(const IntBasis& ib, double primtol, double period, int rc
                         PrimPair pp;
                         pp.zeta = z;
                         pp.h = 0.5 / z;
+                        pp.a2 = 2.0 * al;
                         pp.K = cc * e * c0 / z;
                         pp.Px = (al * axs + be * bxs) / z;
                         pp.Py = (al * A.y + be * B.y) / z;

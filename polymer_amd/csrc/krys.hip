@@ -402,6 +402,7 @@ static PrimPair host_prim_pair(double a, const double* A, double b, const double
     PrimPair q;
     q.zeta = a + b;
     q.h = 0.5 / q.zeta;
+    q.a2 = 2.0 * a;
     const double d2 = (A[0] - B[0]) * (A[0] - B[0]) + (A[1] - B[1]) * (A[1] - B[1]) + (A[2] - B[2]) * (A[2] - B[2]);
     q.K = std::sqrt(2.0) * std::pow(3.141592653589793, 1.25) * std::exp(-a * b / q.zeta * d2) / q.zeta;
     q.Px = (a * A[0] + b * B[0]) / q.zeta;

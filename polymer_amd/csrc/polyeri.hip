@@ -4156,7 +4156,7 @@ int polyeri_set_direct(polyeri_ctx* ctx, int direct) {
 // src/pfourindexgradient.f90:1-1478, molecule): kgrad.hip
 // ---------------------------------------------------------------------------
 struct GradHost {
-    std::vector<int> L, atom, f0, p0, np, pa, pb;
+    std::vector<int> L, atom, f0, p0, np, pa, pb, pp0, pn;
     std::vector<double> xyz, alpha, coef, D, dsh;
     int seg[NPAIRCLASS + 1];
 };
@@ -4218,6 +4218,31 @@ static int grad_host_arrays(const IntBasis& ib, const RefBasis& rb, const double
     return 0;
 }
 
+// Primitive pairs of the sorted pairs in the table of build_pairs, whose
+// pairs are the same shells in the same order (higher L first); qp (optional):
+// their bounds Q.  A pair without primitive pairs above the threshold has none.
+static int grad_pair_prims(const std::vector<PairInfo>& pairs, const std::vector<double>* Q, GradHost& h,
+                           std::vector<double>* qp) {
+    const long long nsh = (long long)h.L.size();
+    std::unordered_map<long long, int> at;
+    at.reserve(pairs.size() * 2);
+    for (size_t i = 0; i < pairs.size(); ++i) at[pairs[i].a * nsh + pairs[i].b] = (int)i;
+    h.pp0.assign(h.pa.size(), 0);
+    h.pn.assign(h.pa.size(), 0);
+    if (qp) qp->assign(h.pa.size(), 0.0);
+    size_t found = 0;
+    for (size_t t = 0; t < h.pa.size(); ++t) {
+        const auto it = at.find(h.pa[t] * nsh + h.pb[t]);
+        if (it == at.end()) continue;
+        ++found;
+        h.pp0[t] = pairs[it->second].prim_off;
+        h.pn[t] = pairs[it->second].nprim;
+        if (qp) (*qp)[t] = (*Q)[it->second];
+    }
+    if (found != pairs.size()) return fail(POLYERI_E_BASIS, "eri gradient: shell pair order differs");
+    return 0;
+}
+
 static int grad_check(polyeri_ctx* ctx, const double* p_c, double* grad, const char* who) {
     if (!ctx || !p_c || !grad) return fail(POLYERI_E_ARG, std::string(who) + ": null argument");
     if (ctx->pbc) return fail(POLYERI_E_ARG, std::string(who) + ": molecular contexts only");
@@ -4233,63 +4258,50 @@ int polyeri_eri_gradient(polyeri_ctx* ctx, const double* p_c, double hfexchange,
     if ((rc = grad_host_arrays(ctx->ib, ctx->rb, p_c, h))) return rc;
     const int nsh = (int)h.L.size(), natom = ctx->rb.natom, nbf = ctx->ib.nbf;
     const size_t npair = h.pa.size();
-    DevBuf buf;
-    int *dL, *dAt, *dF0, *dP0, *dNp, *dPa, *dPb;
-    double *dXyz, *dAl, *dCo, *dD, *dDsh, *dQp, *dG;
-    if ((rc = buf.get(&dL, nsh)) || (rc = buf.get(&dAt, nsh)) || (rc = buf.get(&dF0, nsh)) ||
-        (rc = buf.get(&dP0, nsh)) || (rc = buf.get(&dNp, nsh)) || (rc = buf.get(&dXyz, 3 * (size_t)nsh)) ||
-        (rc = buf.get(&dAl, h.alpha.size())) || (rc = buf.get(&dCo, h.coef.size())) ||
-        (rc = buf.get(&dD, h.D.size())) || (rc = buf.get(&dDsh, h.dsh.size())) || (rc = buf.get(&dQp, npair)) ||
-        (rc = buf.get(&dG, 3 * (size_t)natom)) || (rc = buf.get(&dPa, npair)) || (rc = buf.get(&dPb, npair)))
-        return rc;
-    hipStream_t s = ctx->stream;
-    HIPCHK(hipMemcpyAsync(dL, h.L.data(), nsh * sizeof(int), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dAt, h.atom.data(), nsh * sizeof(int), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dF0, h.f0.data(), nsh * sizeof(int), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dP0, h.p0.data(), nsh * sizeof(int), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dNp, h.np.data(), nsh * sizeof(int), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dXyz, h.xyz.data(), h.xyz.size() * 8, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dAl, h.alpha.data(), h.alpha.size() * 8, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dCo, h.coef.data(), h.coef.size() * 8, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dD, h.D.data(), h.D.size() * 8, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dDsh, h.dsh.data(), h.dsh.size() * 8, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_fill, dim3(nblk(3 * (size_t)natom)), dim3(256), 0, s, dG, 3 * (size_t)natom, 0.0);
     // pair bounds: the context's Schwarz bounds Q_ab = sqrt(max |(ab|ab)|) of
-    // the same shell pairs (pairs the context dropped by primitive screening: 0)
-    std::vector<double> qp(npair, 0.0);
-    {
-        std::unordered_map<long long, double> qmap;
-        qmap.reserve(ctx->pairs.size() * 2);
-        for (size_t i = 0; i < ctx->pairs.size(); ++i) {
-            const int a = ctx->pairs[i].a, b = ctx->pairs[i].b;
-            qmap[(long long)std::min(a, b) * nsh + std::max(a, b)] = ctx->Q[i];
-        }
-        for (size_t t = 0; t < npair; ++t) {
-            auto it = qmap.find((long long)std::min(h.pa[t], h.pb[t]) * nsh + std::max(h.pa[t], h.pb[t]));
-            if (it != qmap.end()) qp[t] = it->second;
-        }
-    }
-    // only the quartets with Q_ab Q_cd >= tol are launched (pairs reordered
-    // by bound inside each class and primitive count)
-    const bool sorted = polyeri_grad_sort_pairs(h.pa.data(), h.pb.data(), qp.data(), h.np.data(), h.seg);
+    // the same shell pairs; only the quartets with Q_ab Q_cd >= tol are
+    // launched (pairs reordered by bound inside each class and primitive count)
+    std::vector<double> qp;
+    if ((rc = grad_pair_prims(ctx->pairs, &ctx->Q, h, &qp))) return rc;
+    const bool sorted = polyeri_grad_sort_pairs(h.pa.data(), h.pb.data(), qp.data(), h.pp0.data(), h.pn.data(), h.seg);
     GradChunks ch;
-    unsigned long long* dOff = nullptr;
-    int* dIj = nullptr;
-    if (sorted) {
-        polyeri_grad_chunks(h.pa.data(), h.pb.data(), h.np.data(), qp.data(), h.seg, ctx->opts.schwarz_tol, ch);
-        if ((rc = buf.get(&dOff, ch.off.size())) || (rc = buf.get(&dIj, std::max<size_t>(ch.ij.size(), 1)))) return rc;
-        HIPCHK(hipMemcpyAsync(dOff, ch.off.data(), ch.off.size() * 8, hipMemcpyHostToDevice, s));
-        if (!ch.ij.empty())
-            HIPCHK(hipMemcpyAsync(dIj, ch.ij.data(), ch.ij.size() * sizeof(int), hipMemcpyHostToDevice, s));
-    }
-    HIPCHK(hipMemcpyAsync(dPa, h.pa.data(), npair * sizeof(int), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dPb, h.pb.data(), npair * sizeof(int), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dQp, qp.data(), npair * sizeof(double), hipMemcpyHostToDevice, s));
-    GradArgs g{nsh, natom, nbf, (int)npair, {0}, dL, dAt, dF0, dP0, dNp, dPa, dPb, dXyz, dAl, dCo, dD, dDsh,
-               nullptr, ctx->opts.schwarz_tol, hfexchange, ctx->opts.prim_tol};
+    polyeri_grad_chunks(qp.data(), h.pn.data(), h.seg, ctx->opts.schwarz_tol, sorted, true, ch);
+    DevBuf buf;
+    int *dAt, *dF0, *dPa, *dPb, *dPp, *dPn, *dIj;
+    double *dXyz, *dD, *dDsh, *dQp, *dG;
+    unsigned long long* dOff;
+    hipStream_t s = ctx->stream;
+    auto put = [&](auto** d, const auto& v) -> int {
+        int e = buf.get(d, std::max<size_t>(v.size(), 1));
+        if (e || v.empty()) return e;
+        HIPCHK(hipMemcpyAsync(*d, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, s));
+        return 0;
+    };
+    if ((rc = put(&dAt, h.atom)) || (rc = put(&dF0, h.f0)) || (rc = put(&dXyz, h.xyz)) || (rc = put(&dD, h.D)) ||
+        (rc = put(&dDsh, h.dsh)) || (rc = put(&dPa, h.pa)) || (rc = put(&dPb, h.pb)) || (rc = put(&dPp, h.pp0)) ||
+        (rc = put(&dPn, h.pn)) || (rc = put(&dQp, qp)) || (rc = put(&dOff, ch.off)) || (rc = put(&dIj, ch.ij)) ||
+        (rc = buf.get(&dG, 3 * (size_t)natom)))
+        return rc;
+    hipLaunchKernelGGL(k_fill, dim3(nblk(3 * (size_t)natom)), dim3(256), 0, s, dG, 3 * (size_t)natom, 0.0);
+    GradArgs g{nsh, natom, nbf, (int)npair, {0}, dAt, dF0, dPa, dPb, dPp, dPn, ctx->d_prims, dXyz, dD, dDsh, dQp,
+               ctx->opts.schwarz_tol, hfexchange};
     std::copy(h.seg, h.seg + NPAIRCLASS + 1, g.seg);
-    if (polyeri_grad_launch(g, dQp, dG, s, true, sorted ? &ch : nullptr, dOff, dIj))
+    // the launches only add to dG: four streams side by side, joined below
+    HIPCHK(hipEventRecord(ctx->ev_fork, s));
+    hipStream_t st[kBranches] = {s};
+    for (int i = 0; i < kBranches - 1; ++i) {
+        st[i + 1] = ctx->side[i];
+        HIPCHK(hipStreamWaitEvent(st[i + 1], ctx->ev_fork, 0));
+    }
+    const int lrc = polyeri_grad_launch(g, dG, st, kBranches, ch, dOff, dIj);
+    for (int i = 0; i < kBranches - 1; ++i) {      // also after a failed launch: the buffers end with this call
+        HIPCHK(hipEventRecord(ctx->ev_join[i], st[i + 1]));
+        HIPCHK(hipStreamWaitEvent(s, ctx->ev_join[i], 0));
+    }
+    if (lrc) {
+        (void)hipStreamSynchronize(s);
         return fail(POLYERI_E_HIP, "polyeri_eri_gradient: launch failed");
+    }
     HIPCHK(hipMemcpyAsync(grad, dG, 3 * (size_t)natom * 8, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     for (int i = 0; i < 3 * natom; ++i)
@@ -4321,11 +4333,17 @@ int polyeri_eri_gradient_host(int npgs, int ncgs, const int* pax, const int* pay
     if (extract_shells(rb, ib, err)) return fail(POLYERI_E_BASIS, err);
     GradHost h;
     if (int rc = grad_host_arrays(ib, rb, p_c, h)) return rc;
-    GradArgs g{(int)h.L.size(), natom, ib.nbf, (int)h.pa.size(), {0}, h.L.data(), h.atom.data(), h.f0.data(),
-               h.p0.data(), h.np.data(), h.pa.data(), h.pb.data(), h.xyz.data(), h.alpha.data(), h.coef.data(),
-               h.D.data(), h.dsh.data(), nullptr, schwarz_tol, hfexchange, 1e-20};
+    const double ptol = 1e-20;
+    std::vector<PairInfo> pairs;
+    std::vector<PrimPair> prims;
+    build_pairs(ib, ptol, pairs, prims);
+    if (int rc = grad_pair_prims(pairs, nullptr, h, nullptr)) return rc;
+    GradArgs g{(int)h.L.size(), natom, ib.nbf, (int)h.pa.size(), {0}, h.atom.data(), h.f0.data(), h.pa.data(),
+               h.pb.data(), h.pp0.data(), h.pn.data(), prims.data(), h.xyz.data(), h.D.data(), h.dsh.data(), nullptr,
+               schwarz_tol, hfexchange};
+    const GradShells gs{h.L.data(), h.p0.data(), h.np.data(), h.xyz.data(), h.alpha.data(), h.coef.data(), ptol};
     std::copy(h.seg, h.seg + NPAIRCLASS + 1, g.seg);
-    return polyeri_grad_host(g, grad) ? fail(POLYERI_E_ARG, "polyeri_eri_gradient_host failed") : 0;
+    return polyeri_grad_host(g, gs, grad) ? fail(POLYERI_E_ARG, "polyeri_eri_gradient_host failed") : 0;
 }
 
 // One-electron and nuclear parts of the nuclear gradient (OVERLAP_KINETIC(1),
