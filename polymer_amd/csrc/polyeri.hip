@@ -1720,22 +1720,10 @@ static int jk_enqueue(polyeri_ctx* c, const double* d_pc, double* d_jc, double* 
     std::vector<int> branch(c->work.size(), 0);
     hipStream_t main = c->stream;
     if (fork) {
-        std::vector<int> order(c->work.size());
-        for (size_t w = 0; w < order.size(); ++w) order[w] = (int)w;
         const bool timed = std::all_of(c->work.begin(), c->work.end(),
                                        [](const ClassPairWork& x) { return x.nwork <= 0 || x.est_ms > 0; });
-        auto cost = [&](int w) { return timed ? c->work[w].est_ms : c->work[w].flops; };
-        std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost(a) > cost(b); });
-        double load[kBranches] = {};
-        for (int w : order) {
-            int bmin = 0;
-            for (int i = 1; i < kBranches; ++i)
-                if (load[i] < load[bmin]) bmin = i;
-            branch[w] = bmin;
-            load[bmin] += cost(w);
-        }
-        HIPCHK(hipEventRecord(c->ev_fork, main));
-        for (int i = 0; i < kBranches - 1; ++i) HIPCHK(hipStreamWaitEvent(c->side[i], c->ev_fork, 0));
+        branch = deal_branches(c->work.size(), [&](int w) { return timed ? c->work[w].est_ms : c->work[w].flops; });
+        if (int frc = fork_branches(c)) return frc;
     }
     int rc = 0;
     for (size_t w = 0; w < c->work.size() && !rc; ++w) {
@@ -1758,11 +1746,10 @@ static int jk_enqueue(polyeri_ctx* c, const double* d_pc, double* d_jc, double* 
         }
         c->stream = main;
     }
-    if (fork)   // join every branch, also after a failed launch (capture must end joined)
-        for (int i = 0; i < kBranches - 1; ++i) {
-            HIPCHK(hipEventRecord(c->ev_join[i], c->side[i]));
-            HIPCHK(hipStreamWaitEvent(main, c->ev_join[i], 0));
-        }
+    if (fork) {   // join every branch, also after a failed launch (capture must end joined)
+        const int jrc = join_branches(c);
+        if (!rc) rc = jrc;
+    }
     if (rc) return rc;
     if (c->profiling) HIPCHK(hipEventRecord(c->ev[c->work.size()], c->stream));
     hipLaunchKernelGGL(k_fill, dim3(nblk(c2)), dim3(256), 0, c->stream, d_jc, c2, 0.0);
@@ -1776,6 +1763,58 @@ static int jk_enqueue(polyeri_ctx* c, const double* d_pc, double* d_jc, double* 
 // One J/K build.  Without per-class profiling the kernel sequence is
 // captured once per (density, J, K, screening) combination into a HIP graph
 // and replayed; the timing events stay outside the graph.
+// Independent launches of one call over kBranches streams: the context's own
+// and the device's side streams, which wait for what is enqueued on it so far
+// (fork_branches) and which it waits for afterwards (join_branches).
+static int fork_branches(polyeri_ctx* c) {
+    HIPCHK(hipEventRecord(c->ev_fork, c->stream));
+    for (int i = 0; i < kBranches - 1; ++i) HIPCHK(hipStreamWaitEvent(c->side[i], c->ev_fork, 0));
+    return 0;
+}
+static int join_branches(polyeri_ctx* c) {
+    for (int i = 0; i < kBranches - 1; ++i) {
+        HIPCHK(hipEventRecord(c->ev_join[i], c->side[i]));
+        HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join[i], 0));
+    }
+    return 0;
+}
+// The branch of each of n launches: costliest first, to the least loaded one.
+template <typename Cost>
+static std::vector<int> deal_branches(size_t n, Cost cost) {
+    std::vector<int> branch(n, 0), order(n);
+    for (size_t w = 0; w < n; ++w) order[w] = (int)w;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost(a) > cost(b); });
+    double load[kBranches] = {};
+    for (int w : order) {
+        int bmin = 0;
+        for (int i = 1; i < kBranches; ++i)
+            if (load[i] < load[bmin]) bmin = i;
+        branch[w] = bmin;
+        load[bmin] += cost(w);
+    }
+    return branch;
+}
+// Runs launch(list) for every work list on its branch (all on the context's
+// stream where fork is false); the kernels go to c->stream.
+template <typename Launch>
+static int launch_lists(polyeri_ctx* c, bool fork, Launch launch) {
+    const std::vector<int> branch =
+        fork ? deal_branches(c->work.size(), [&](int w) { return c->work[w].flops; }) : std::vector<int>();
+    int rc = fork ? fork_branches(c) : 0;
+    if (rc) return rc;
+    hipStream_t main = c->stream;
+    for (size_t w = 0; w < c->work.size() && !rc; ++w) {
+        if (fork && branch[w]) c->stream = c->side[branch[w] - 1];
+        rc = launch(w);
+        c->stream = main;
+    }
+    if (fork) {                                   // joined also after a failed launch
+        const int jrc = join_branches(c);
+        if (!rc) rc = jrc;
+    }
+    return rc;
+}
+
 // J/K from the stored records (DIRECT .F.) into the reference-layout
 // blocks d_jc / d_kc (ncell blocks: 1 for a molecule).
 static int jk_stored(polyeri_ctx* c, const double* d_pc, double* d_jc, double* d_kc) {
@@ -1932,12 +1971,13 @@ static int jk_device_cells(polyeri_ctx* c, const double* d_pc, double* d_jc, dou
     hipLaunchKernelGGL(k_fill, dim3(nblk(nj)), dim3(256), 0, c->stream, c->d_Kc, nj, 0.0);
     HIPCHK(hipGetLastError());
     const long long n3 = 2LL * c->cel2 + 1;
-    for (size_t w = 0; w < c->work.size(); ++w) {
-        const ClassPairWork& cw = c->work[w];
+    // the lists only add to the J/K cells; profiled builds stay on one stream
+    // (per-list events between the launches)
+    int rc = launch_lists(c, !c->profiling, [&](size_t w) -> int {
         if (c->profiling) HIPCHK(hipEventRecord(c->ev[w], c->stream));
-        int rc = launch_class_pbc(c, cw, cw.nwork * n3);
-        if (rc) return rc;
-    }
+        return launch_class_pbc(c, c->work[w], c->work[w].nwork * n3);
+    });
+    if (rc) return rc;
     if (c->profiling) HIPCHK(hipEventRecord(c->ev[c->work.size()], c->stream));
     hipLaunchKernelGGL(k_fill, dim3(nblk(c2 * ncell)), dim3(256), 0, c->stream, d_jc, c2 * ncell, 0.0);
     hipLaunchKernelGGL(k_fill, dim3(nblk(c2 * ncell)), dim3(256), 0, c->stream, d_kc, c2 * ncell, 0.0);
@@ -2060,16 +2100,16 @@ static int tensor_device(polyeri_ctx* c, double* d_t, bool packed = false) {
         return 0;
     }
     c->tpack = packed;
-    for (const ClassPairWork& cw : c->work) {
+    // each integral has one producer, so the lists run side by side
+    int rc = launch_lists(c, true, [&](size_t w) {
         // lists with a generally contracted form of shell-pair groups: one
         // primitive loop per group quartet for all its member quartets
         const bool gc = cw.gc.nwork > 0 && cw.gc.kind == 0;
-        int rc = gc ? launch_gc(c, cw, cw.gc_block, nullptr, d_t)
-                    : launch_class(c, MODE_TENSOR, cw.la, cw.lb, cw.lc, cw.ld, cw.d_bra, cw.d_ket, cw.d_row,
-                                   cw.nrows, cw.nwork, d_t, cw.d_rb, cw.d_bstart, cw.nbucket, cw.d_rf, nullptr,
-                                   nullptr, LaunchCfg(), cw.d_bsoa);
-        if (rc) { c->tpack = 0; return rc; }
-    }
+        return gc ? launch_gc(c, cw, cw.gc_block, nullptr, d_t)
+                  : launch_class(c, MODE_TENSOR, cw.la, cw.lb, cw.lc, cw.ld, cw.d_bra, cw.d_ket, cw.d_row, cw.nrows,
+                                 cw.nwork, d_t, cw.d_rb, cw.d_bstart, cw.nbucket, cw.d_rf, nullptr, nullptr,
+                                 LaunchCfg(), cw.d_bsoa);
+    });
     c->tpack = 0;
     return 0;
 }
@@ -2144,7 +2184,7 @@ int polyeri_get_stats(polyeri_ctx* ctx, polyeri_stats* st) {
         }
         st->class_l[i] = w.la * 1000 + w.lb * 100 + w.lc * 10 + w.ld;
     }
-    return 0;
+    return rc;
 }
 
 // ---------------------------------------------------------------------------
@@ -2162,6 +2202,7 @@ static void lu_solve(int n, const std::vector<double>& A0, const std::vector<dou
         double m = 0;
         for (int j = 0; j < n; ++j) m = std::max(m, std::fabs(A[i + n * j]));
         sc[i] = m > 0 ? 1.0 / m : 1.0;
+        const ClassPairWork& cw = c->work[w];
     }
     for (int k = 0; k < n; ++k) {
         int p = k;
@@ -3577,11 +3618,8 @@ static int tensor_device_cells(polyeri_ctx* c, double* dT, size_t nt) {
     hipLaunchKernelGGL(k_fill, dim3(nblk(nt)), dim3(256), 0, c->stream, dT, nt, 0.0);
     HIPCHK(hipGetLastError());
     const long long n3 = 2LL * c->cel2 + 1;
-    for (const ClassPairWork& cw : c->work) {
-        int rc = launch_class_pbc(c, cw, cw.nwork * n3, dT);
-        if (rc) return rc;
-    }
-    return 0;
+    // each integral has one producer
+    return launch_lists(c, true, [&](size_t w) { return launch_class_pbc(c, c->work[w], c->work[w].nwork * n3, dT); });
 }
 
 // CO(k) (reference order, complex, column-major per k) -> planar internal
@@ -4287,17 +4325,11 @@ int polyeri_eri_gradient(polyeri_ctx* ctx, const double* p_c, double hfexchange,
                ctx->opts.schwarz_tol, hfexchange};
     std::copy(h.seg, h.seg + NPAIRCLASS + 1, g.seg);
     // the launches only add to dG: four streams side by side, joined below
-    HIPCHK(hipEventRecord(ctx->ev_fork, s));
+    if ((rc = fork_branches(ctx))) return rc;
     hipStream_t st[kBranches] = {s};
-    for (int i = 0; i < kBranches - 1; ++i) {
-        st[i + 1] = ctx->side[i];
-        HIPCHK(hipStreamWaitEvent(st[i + 1], ctx->ev_fork, 0));
-    }
+    for (int i = 0; i < kBranches - 1; ++i) st[i + 1] = ctx->side[i];
     const int lrc = polyeri_grad_launch(g, dG, st, kBranches, ch, dOff, dIj);
-    for (int i = 0; i < kBranches - 1; ++i) {      // also after a failed launch: the buffers end with this call
-        HIPCHK(hipEventRecord(ctx->ev_join[i], st[i + 1]));
-        HIPCHK(hipStreamWaitEvent(s, ctx->ev_join[i], 0));
-    }
+    if ((rc = join_branches(ctx))) return rc;      // also after a failed launch: the buffers end with this call
     if (lrc) {
         (void)hipStreamSynchronize(s);
         return fail(POLYERI_E_HIP, "polyeri_eri_gradient: launch failed");
