@@ -126,14 +126,19 @@ unsigned grid_of(long long n) {
     return (unsigned)std::max<long long>(1, std::min<long long>(b, 4096));
 }
 
+// Work buffers from the library's pool, given back once the stream is done.
 struct Dev {
     std::vector<void*> ptrs;
+    hipStream_t s;
+    explicit Dev(hipStream_t s) : s(s) {}
+    Dev(const Dev&) = delete;
     ~Dev() {
-        for (void* p : ptrs) (void)hipFree(p);
+        if (!ptrs.empty()) (void)hipStreamSynchronize(s);
+        for (void* p : ptrs) polyeri_work_put(p);
     }
     double* get(size_t n) {
         void* p = nullptr;
-        if (hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(double)) != hipSuccess) return nullptr;
+        if (polyeri_work_get(&p, std::max<size_t>(n, 1) * sizeof(double))) return nullptr;
         ptrs.push_back(p);
         return (double*)p;
     }
@@ -364,7 +369,7 @@ int polyeri_cc_solve(const double* dG, int nmo, int no_, const double* eps, int 
     }
     ndiis = std::max(1, std::min(ndiis, 16));
     const long long o2v2 = no * no * nv * nv, n1 = no * nv, n12 = n1 + o2v2;
-    Dev dv;
+    Dev dv(s);
     Engine E{s, no, nv, nullptr, nullptr, nullptr, nullptr, nullptr, err};
     double *ovov, *oovv, *ovvo, *ovoo, *ovvv, *O2, *V2, *L, *Lp, *dEps;
     double *T, *Tn, *R, *tau, *tauF, *tk, *tl, *x, *u;

@@ -463,6 +463,7 @@ struct ScfArena {
 
 struct polyeri_ctx {
     int tpack = 0;                 // MODE_TENSOR launches write the pair-packed tensor
+    bool counted = false;          // among the work pool's live contexts
     RefBasis rb;
     IntBasis ib;
     std::vector<PairInfo> pairs;
@@ -586,10 +587,105 @@ static int ensure_onee_device(polyeri_ctx* c) {
     return 0;
 }
 
+// Work buffers of single calls (MP2, CC, gradient, k-point SCF), kept between
+// calls: mapping and unmapping gigabytes on each call took longer than the
+// call ((H2O)8 cc-pVDZ MP2: 17 ms of kernels, 130 to 270 ms with hipMalloc and
+// hipFree of its 9 GB in a process that holds other allocations).  A block is
+// handed out only while it is in use by nobody (mutex; the caller waits for
+// its streams before it gives a block back).  At most a quarter of the
+// device's memory is kept idle, all of it goes back when the device's last
+// context ends or an allocation fails.
+struct WorkPool {
+    struct Block {
+        void* p;
+        size_t bytes;
+        int device;
+    };
+    std::mutex mu;
+    std::vector<Block> idle, used;
+    std::vector<int> contexts;            // live contexts per device
+
+    size_t idle_bytes(int device) {
+        size_t n = 0;
+        for (const Block& b : idle) n += b.device == device ? b.bytes : 0;
+        return n;
+    }
+    void release(int device) {            // with mu held
+        for (size_t i = idle.size(); i-- > 0;)
+            if (idle[i].device == device) {
+                (void)hipFree(idle[i].p);
+                idle.erase(idle.begin() + i);
+            }
+    }
+    hipError_t get(void** p, size_t bytes) {
+        int device = 0;
+        hipError_t e = hipGetDevice(&device);
+        if (e != hipSuccess) return e;
+        std::lock_guard<std::mutex> lk(mu);
+        size_t best = idle.size();        // the smallest idle block that holds it and is not twice too large
+        for (size_t i = 0; i < idle.size(); ++i)
+            if (idle[i].device == device && idle[i].bytes >= bytes && idle[i].bytes / 2 <= bytes + 32768 &&
+                (best == idle.size() || idle[i].bytes < idle[best].bytes))
+                best = i;
+        if (best < idle.size()) {
+            used.push_back(idle[best]);
+            idle.erase(idle.begin() + best);
+        } else {
+            void* q = nullptr;
+            e = hipMalloc(&q, bytes);
+            if (e != hipSuccess) {
+                (void)hipGetLastError();
+                release(device);
+                e = hipMalloc(&q, bytes);
+            }
+            if (e != hipSuccess) return e;
+            used.push_back({q, bytes, device});
+        }
+        *p = used.back().p;
+        return hipSuccess;
+    }
+    void put(void* p) {
+        std::lock_guard<std::mutex> lk(mu);
+        for (size_t i = 0; i < used.size(); ++i) {
+            if (used[i].p != p) continue;
+            const Block b = used[i];
+            used.erase(used.begin() + i);
+            size_t freeb = 0, total = 0;
+            if (hipMemGetInfo(&freeb, &total) == hipSuccess && idle_bytes(b.device) + b.bytes <= total / 4)
+                idle.push_back(b);
+            else
+                (void)hipFree(b.p);
+            return;
+        }
+    }
+    void context(int device, int step) {
+        std::lock_guard<std::mutex> lk(mu);
+        if ((int)contexts.size() <= device) contexts.resize(device + 1, 0);
+        contexts[device] += step;
+        if (contexts[device] <= 0) release(device);
+    }
+};
+// never destroyed: a context may end after the static objects
+static WorkPool& work_pool() {
+    static WorkPool* pool = new WorkPool;
+    return *pool;
+}
+int polyeri_work_get(void** p, size_t bytes) { return work_pool().get(p, bytes) == hipSuccess ? 0 : -1; }
+void polyeri_work_put(void* p) { work_pool().put(p); }
+
 template <typename T>
 static int dalloc(T** p, size_t n) {
     if (n == 0) n = 1;
     hipError_t e = hipMalloc((void**)p, n * sizeof(T));
+    if (e != hipSuccess) {                // idle work buffers may be in the way
+        (void)hipGetLastError();
+        int device = 0;
+        if (hipGetDevice(&device) == hipSuccess) {
+            std::lock_guard<std::mutex> lk(work_pool().mu);
+            work_pool().release(device);
+        }
+        e = hipMalloc((void**)p, n * sizeof(T));
+    }
     if (e != hipSuccess) return fail(POLYERI_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     return 0;
 }
@@ -913,6 +1009,7 @@ static void free_ctx(polyeri_ctx* c) {
         if (e) (void)hipEventDestroy(e);
     if (c->blas) rocblas_destroy_handle(c->blas);
     drop_graphs(c);
+    if (c->counted) work_pool().context(c->device, -1);
     delete c;
 }
 
@@ -1115,6 +1212,8 @@ static int build_ctx(polyeri_ctx* c) {
     int src = 0;
     c->stream = shared_stream(c->device, &src);
     if (src) return src;
+    work_pool().context(c->device, 1);
+    c->counted = true;
     HIPCHK(hipEventCreate(&c->ev0));
     HIPCHK(hipEventCreate(&c->ev1));
     if ((src = shared_side_streams(c->device, c->side))) return src;
@@ -2274,12 +2373,21 @@ static int form_c2s(const RefBasis& rb, int spherical, std::vector<double>& c2s)
 
 struct DevBuf {
     std::vector<void*> ptrs;
-    ~DevBuf() { for (void* p : ptrs) (void)hipFree(p); }
+    hipStream_t stream;
+    explicit DevBuf(hipStream_t s) : stream(s) {}
+    DevBuf(const DevBuf&) = delete;
+    ~DevBuf() {
+        if (!ptrs.empty()) (void)hipStreamSynchronize(stream);   // also where the call ended early
+        for (void* p : ptrs) work_pool().put(p);
+    }
     template <typename T>
     int get(T** p, size_t n) {
-        int rc = dalloc(p, n);
-        if (!rc) ptrs.push_back(*p);
-        return rc;
+        void* q = nullptr;
+        const hipError_t e = work_pool().get(&q, std::max<size_t>(n, 1) * sizeof(T));
+        if (e != hipSuccess) return fail(POLYERI_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+        ptrs.push_back(q);
+        *p = static_cast<T*>(q);
+        return 0;
     }
 };
 
@@ -2531,7 +2639,7 @@ int polyeri_scf(polyeri_ctx* ctx, const polyeri_scf_opts* o, double* p_c, double
         std::vector<int> keep;
         for (int j = 0; j < nc; ++j) if (e[j] > o->lindep) keep.push_back(j);
         if (keep.empty()) return fail(POLYERI_E_ARG, "no linearly independent functions");
-        DevBuf once;   // not from the arena, so its slots keep their sizes from call to call
+        DevBuf once(s);   // not from the arena, so its slots keep their sizes from call to call
         int* dKeep;
         if ((rc = once.get(&dKeep, keep.size()))) return rc;
         HIPCHK(hipMemcpy(dKeep, keep.data(), keep.size() * sizeof(int), hipMemcpyHostToDevice));
@@ -2950,7 +3058,7 @@ static int mp2_energy(polyeri_ctx* ctx, const double* co, const double* eps, int
     const size_t n4 = packed ? npk * n * n : (size_t)n * n * n * n;
     if (packed && (npk * n > (size_t)INT_MAX || (size_t)n * nvp * nop > (size_t)INT_MAX))
         return fail(POLYERI_E_ARG, "polyeri_mp2_energy: basis too large");
-    DevBuf buf;
+    DevBuf buf(ctx->stream);
     double *dTen, *dCO, *dC, *dX1, *dX2, *dX3, *dT4, *dEps, *dAcc, *dQ, *dY = nullptr;
     // occupied-side indices first: the largest intermediate is nop n^3 (full
     // tensor) or nop n npk (packed)
@@ -3172,7 +3280,7 @@ static int mo_tensor_device(polyeri_ctx* ctx, const double* co, int lo, int hi, 
 int polyeri_mo_integrals(polyeri_ctx* ctx, const double* co, int lo, int hi, double* g) {
     if (!ctx || !co || !g) return fail(POLYERI_E_ARG, "polyeri_mo_integrals: null argument");
     HIPCHK(hipSetDevice(ctx->device));
-    DevBuf buf;
+    DevBuf buf(ctx->stream);
     double* dG = nullptr;
     int rc = mo_tensor_device(ctx, co, lo, hi, buf, &dG, nullptr, nullptr);
     if (rc) return rc;
@@ -3196,7 +3304,7 @@ int polyeri_cc(polyeri_ctx* ctx, const char* method, const double* co, const dou
     if (!(conv > 0.0) || maxiter < 1) return fail(POLYERI_E_ARG, "polyeri_cc: bad convergence request");
     auto t0 = std::chrono::steady_clock::now();
     HIPCHK(hipSetDevice(ctx->device));
-    DevBuf buf;
+    DevBuf buf(ctx->stream);
     double* dG = nullptr;
     double mst = 0.0, msx = 0.0;
     int rc = mo_tensor_device(ctx, co, icore, hi, buf, &dG, &mst, &msx);
@@ -3393,7 +3501,7 @@ int polyeri_scf_periodic(polyeri_ctx* ctx, const polyeri_scf_opts* o, int kvc, d
     double enuc = 0.0;
     one_electron_cells(ctx, Sh, Th, Nh, enuc);
     if ((rc = form_c2s(ctx->rb, o->spherical, c2s))) return rc;
-    DevBuf buf;
+    DevBuf buf(ctx->stream);
     double *dS, *dT, *dN, *dF, *dP, *dPout, *dE, *dOcc, *dSE;
     rocblas_double_complex *dSk, *dFk, *dW1, *dW2, *dX, *dC2S, *dCk;
     int* dInfo;
@@ -3826,10 +3934,20 @@ static int mp2_periodic(polyeri_ctx* ctx, int kvc, const double* co, const doubl
                         sizeof(double2) * (size_t)nc * nc * nk;
     size_t freeb = 0, totalb = 0;
     HIPCHK(hipMemGetInfo(&freeb, &totalb));
+    {
+        std::lock_guard<std::mutex> lk(work_pool().mu);   // idle work buffers are reused or released
+        freeb += work_pool().idle_bytes(ctx->device);
+    }
     if (need > freeb - freeb / 16)
         return fail(POLYERI_E_NOMEM, "polyeri_mp2_energy_periodic: " + std::to_string(need >> 20) +
                                          " MiB of transform buffers exceed free device memory");
-    DevBuf buf;
+    // k-points whose first quarter is one product: the tensor is read once for
+    // all of them; at most half of what is left of the free memory, and an
+    // eighth of the device's, for their TN
+    const size_t more = std::min((freeb - freeb / 16 - need) / 2, totalb / 8) / (16 * (nTN + nB1));
+    const int kgrp = (int)std::min<size_t>(nk, 1 + more);
+    int kfirst = 0;
+    DevBuf buf(ctx->stream);
     double *dT, *dTNr, *dTNi, *dTOKr, *dTOKi, *dTVr, *dTVi, *dTOVr, *dTOVi, *dB1r, *dB1i, *dB2r, *dB2i, *dB3r, *dB3i,
         *dB4r, *dB4i, *dCr, *dCi, *dEps, *dAcc, *dQ = nullptr;
     double2* dCO;
@@ -4304,7 +4422,7 @@ int polyeri_eri_gradient(polyeri_ctx* ctx, const double* p_c, double hfexchange,
     const bool sorted = polyeri_grad_sort_pairs(h.pa.data(), h.pb.data(), qp.data(), h.pp0.data(), h.pn.data(), h.seg);
     GradChunks ch;
     polyeri_grad_chunks(qp.data(), h.pn.data(), h.seg, ctx->opts.schwarz_tol, sorted, true, ch);
-    DevBuf buf;
+    DevBuf buf(ctx->stream);
     int *dAt, *dF0, *dPa, *dPb, *dPp, *dPn, *dIj;
     double *dXyz, *dD, *dDsh, *dQp, *dG;
     unsigned long long* dOff;
