@@ -311,80 +311,172 @@ __global__ void __launch_bounds__(256) k_gemm_bf16x3(GemmArgs g) {
 }
 
 // Planar complex products for the k-point MP2 transform:
-//   C_b = A_b B_b with A = Ar + i Ai (Ai null: A real), B = Br + i Bi,
-//   C = Cr + i Ci, all planes sharing one set of strides.
+//   C = A B with A = Ar + i Ai (Ai null: A real), B = Br + i Bi,
+//   C = Cr + i Ci, all planes sharing one set of strides, k contiguous in A
+//   (A(m, k) = A[m sam + k]) and n in B (B(k, n) = B[k sbk + n]).
 // Real and imaginary parts accumulate in two MFMA accumulators:
 //   Cr += Ar Br - Ai Bi,  Ci += Ar Bi + Ai Br.
 // Column n of B and C is (n / nci, n % nci), at offset
-// (n / nci) sbo + (n % nci) sbn in B and (n / nci) sco + (n % nci) scn in C,
-// so that several products sharing A run as one (nci = N: plain columns).
+// (n / nci) sbo + (n % nci) in B and (n / nci) sco + (n % nci) scn in C, and
+// row m of C (m / mci, m % mci), at (m / mci) smo + (m % mci) scm, so that
+// several products sharing an operand run as one (nci = N, mci = M: plain).
+// Batches (grid.y) add sA, sB, sC.
 struct ZGemmArgs {
     int M, N, K;
     const double *Ar, *Ai;
-    long sam, sak, sA;
+    long sam, sA;
     const double *Br, *Bi;
-    long sbk, sbn, sB;
+    long sbk, sB;
     double *Cr, *Ci;
     long scm, scn, sC;
     int nci;
     long sbo, sco;
+    int mci;
+    long smo;
 };
+__device__ __forceinline__ long zrow(const ZGemmArgs& g, int m) {
+    return (long)(m / g.mci) * g.smo + (long)(m % g.mci) * g.scm;
+}
+__device__ __forceinline__ long zcol(const ZGemmArgs& g, int n) {
+    return (long)(n / g.nci) * g.sco + (long)(n % g.nci) * g.scn;
+}
 
-// Each wavefront computes NT column tiles of one 16-row strip, so the A
-// value it loads per k step feeds NT (complex: 2 NT or 4 NT) products.
-template <int NT>
-__global__ void __launch_bounds__(256) k_zgemm_f64(ZGemmArgs g) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int groups = (g.N + 16 * NT - 1) / (16 * NT);
-    const long tile = (long)blockIdx.x * 4 + wave;
-    const int tm = (int)(tile / groups), tg = (int)(tile % groups);
-    if ((long)tm * 16 >= g.M) return;
-    const long b = blockIdx.y;
-    const bool cplx = g.Ai != nullptr;
-    const long oa = b * g.sA, ob = b * g.sB;
-    const int r = lane & 15, q = lane >> 4;
-    const int m = tm * 16 + r;
-    doublex4 cr[NT], ci[NT];
-    long bcol[NT];
+// LDS-tiled FP64 form: a block of four wavefronts computes 128 rows (32 each)
+// by 16 TNW columns, K eight at a time through two LDS buffers, the next slice
+// in flight while the current one feeds the MFMA units.  The products are
+// tall (10^4 to 10^6 rows, at most a few hundred columns), so the wavefronts
+// split the rows and share the columns, and TNW is the count that leaves
+// fewest padded columns; a row strip's column blocks are neighbours in the
+// grid and read its A from L2.  Without LDS each wavefront loaded A from
+// global memory for its own 16 rows, four k at a time, and waited: the first
+// quarter of (C2H4)3 STO-3G ran at 1.6 TB/s, the second at 40 TF/s.  ROWC:
+// rows of C are contiguous (scm = 1), so the operands swap places and a lane
+// group stores 16 rows of one column as one line.
+template <int TNW, bool CPLX, bool ROWC>
+__global__ void __launch_bounds__(256, 2) k_zgemm_f64(ZGemmArgs g, int nblocks) {
+    constexpr int TMW = 2, BM = 128, BN = 16 * TNW, TK = 8, LA = BM + 8, LB = BN + 8;
+    constexpr int NA = BM * TK / 256, NB = (BN * TK + 255) / 256;
+    __shared__ double As[2][CPLX ? 2 : 1][TK][LA];
+    __shared__ double Bs[2][2][TK][LB];
+    const int n0 = (int)(blockIdx.x % (unsigned)nblocks) * BN;
+    const int m0 = (int)(blockIdx.x / (unsigned)nblocks) * BM;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, r = lane & 15, q = lane >> 4;
+    const long oa = blockIdx.y * g.sA, ob = blockIdx.y * g.sB, oc = blockIdx.y * g.sC;
+    // staging: A element p of this thread is k = t & 7 of row t / 8 + 32 p, B
+    // element p number t + 256 p of the slice in k-major order
+    const int ak = t & 7, am = t >> 3;
+    const double* pa = g.Ar + oa + (long)(m0 + am) * g.sam + ak;
+    const long da = g.Ai - g.Ar;
+    long boff[NB];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        cr[t] = doublex4{0.0, 0.0, 0.0, 0.0};
-        ci[t] = doublex4{0.0, 0.0, 0.0, 0.0};
-        const int n = (tg * NT + t) * 16 + r;
-        bcol[t] = (long)(n / g.nci) * g.sbo + (long)(n % g.nci) * g.sbn;
+    for (int p = 0; p < NB; ++p) {
+        const int e = t + 256 * p, n = n0 + e % BN;
+        boff[p] = n < g.N && e < BN * TK ? ob + (long)(n / g.nci) * g.sbo + n % g.nci + (long)(e / BN) * g.sbk : -1;
     }
-    for (int k0 = 0; k0 < g.K; k0 += 4) {
-        const int k = k0 + q;
-        const bool va = m < g.M && k < g.K;
-        const long ia = oa + m * g.sam + k * g.sak;
-        const double ar = va ? g.Ar[ia] : 0.0;
-        const double ai = (cplx && va) ? g.Ai[ia] : 0.0;
+    double ar[NA], ai[CPLX ? NA : 1], br[NB], bi[NB];
+    auto load = [&](int k0) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const int n = (tg * NT + t) * 16 + r;
-            const bool vb = n < g.N && k < g.K;
-            const long ib = ob + k * g.sbk + bcol[t];
-            const double br = vb ? g.Br[ib] : 0.0, bi = vb ? g.Bi[ib] : 0.0;
-            cr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, cr[t], 0, 0, 0);
-            ci[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, ci[t], 0, 0, 0);
-            if (cplx) {
-                cr[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai, bi, cr[t], 0, 0, 0);
-                ci[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, br, ci[t], 0, 0, 0);
+        for (int p = 0; p < NA; ++p) {
+            const bool in = m0 + am + 32 * p < g.M && k0 + ak < g.K;
+            const double* x = pa + (long)(32 * p) * g.sam + k0;
+            ar[p] = in ? x[0] : 0.0;
+            if constexpr (CPLX) ai[p] = in ? x[da] : 0.0;
+        }
+#pragma unroll
+        for (int p = 0; p < NB; ++p) {
+            const bool in = boff[p] >= 0 && k0 + (t + 256 * p) / BN < g.K;
+            const long x = boff[p] + (long)k0 * g.sbk;
+            br[p] = in ? g.Br[x] : 0.0;
+            bi[p] = in ? g.Bi[x] : 0.0;
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int p = 0; p < NA; ++p) {
+            As[buf][0][ak][am + 32 * p] = ar[p];
+            if constexpr (CPLX) As[buf][1][ak][am + 32 * p] = ai[p];
+        }
+#pragma unroll
+        for (int p = 0; p < NB; ++p) {
+            const int e = t + 256 * p;
+            if (BN * TK % 256 == 0 || e < BN * TK) {
+                Bs[buf][0][e / BN][e % BN] = br[p];
+                Bs[buf][1][e / BN][e % BN] = bi[p];
             }
         }
-    }
-    const long oc = b * g.sC;
+    };
+    doublex4 cr[TMW][TNW], ci[TMW][TNW];
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int i = 0; i < TMW; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = tm * 16 + q + 4 * j, col = (tg * NT + t) * 16 + r;
-            if (row < g.M && col < g.N) {
-                const long ic = oc + row * g.scm + (long)(col / g.nci) * g.sco + (long)(col % g.nci) * g.scn;
-                g.Cr[ic] = cr[t][j];
-                g.Ci[ic] = ci[t][j];
+        for (int j = 0; j < TNW; ++j) cr[i][j] = ci[i][j] = doublex4{0.0, 0.0, 0.0, 0.0};
+    auto mma = [](double a, double b, doublex4 c) {
+        return ROWC ? __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, c, 0, 0, 0)
+                    : __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    };
+    const int wr = wave * TMW * 16;
+    const int nk = (g.K + TK - 1) / TK;
+    load(0);
+    store(0);
+    __syncthreads();
+    for (int it = 0; it < nk; ++it) {
+        const int buf = it & 1;
+        if (it + 1 < nk) load((it + 1) * TK);
+#pragma unroll
+        for (int ks = 0; ks < TK; ks += 4) {
+            double xr[TMW], xi[TMW];
+#pragma unroll
+            for (int i = 0; i < TMW; ++i) {
+                xr[i] = As[buf][0][ks + q][wr + i * 16 + r];
+                if constexpr (CPLX) xi[i] = As[buf][1][ks + q][wr + i * 16 + r];
+            }
+#pragma unroll
+            for (int j = 0; j < TNW; ++j) {
+                const double yr = Bs[buf][0][ks + q][j * 16 + r], yi = Bs[buf][1][ks + q][j * 16 + r];
+#pragma unroll
+                for (int i = 0; i < TMW; ++i) {
+                    cr[i][j] = mma(xr[i], yr, cr[i][j]);
+                    ci[i][j] = mma(xr[i], yi, ci[i][j]);
+                    if constexpr (CPLX) {
+                        cr[i][j] = mma(-xi[i], yi, cr[i][j]);
+                        ci[i][j] = mma(xi[i], yr, ci[i][j]);
+                    }
+                }
             }
         }
+        // the other buffer was read before the previous barrier
+        if (it + 1 < nk) store(buf ^ 1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < TMW; ++i)
+#pragma unroll
+        for (int j = 0; j < TNW; ++j)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                const int row = m0 + wr + i * 16 + (ROWC ? r : q + 4 * x), col = n0 + j * 16 + (ROWC ? q + 4 * x : r);
+                if (row < g.M && col < g.N) {
+                    const long ic = oc + zrow(g, row) + zcol(g, col);
+                    g.Cr[ic] = cr[i][j][x];
+                    g.Ci[ic] = ci[i][j][x];
+                }
+            }
+}
+
+template <int TNW>
+static int launch_zgemm_f64(const ZGemmArgs& g, int nbat, hipStream_t stream) {
+    const long nbk = (g.N + 16 * TNW - 1) / (16 * TNW), mbk = ((long)g.M + 127) / 128;
+    if (mbk * nbk > 0x7fffffffL) return -1;
+    const dim3 grid((unsigned)(mbk * nbk), (unsigned)nbat);
+    if (g.Ai && g.scm == 1)
+        hipLaunchKernelGGL((k_zgemm_f64<TNW, true, true>), grid, dim3(256), 0, stream, g, (int)nbk);
+    else if (g.Ai)
+        hipLaunchKernelGGL((k_zgemm_f64<TNW, true, false>), grid, dim3(256), 0, stream, g, (int)nbk);
+    else if (g.scm == 1)
+        hipLaunchKernelGGL((k_zgemm_f64<TNW, false, true>), grid, dim3(256), 0, stream, g, (int)nbk);
+    else
+        hipLaunchKernelGGL((k_zgemm_f64<TNW, false, false>), grid, dim3(256), 0, stream, g, (int)nbk);
+    return 0;
 }
 
 // acc += x y with x, y given as three BF16 pieces each (six products, small first)
@@ -398,6 +490,8 @@ __device__ __forceinline__ floatx4 mfma_split3(const bf16x4* x, const bf16x4* y,
     return acc;
 }
 
+// Each wavefront computes NT column tiles of one 16-row strip, so the A
+// value it loads per k step feeds NT (complex: 2 NT or 4 NT) products.
 template <int NT>
 __global__ void __launch_bounds__(256) k_zgemm_bf16x3(ZGemmArgs g) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -417,7 +511,7 @@ __global__ void __launch_bounds__(256) k_zgemm_bf16x3(ZGemmArgs g) {
         cr[t] = floatx4{0.f, 0.f, 0.f, 0.f};
         ci[t] = floatx4{0.f, 0.f, 0.f, 0.f};
         const int n = (tg * NT + t) * 16 + r;
-        bcol[t] = (long)(n / g.nci) * g.sbo + (long)(n % g.nci) * g.sbn;
+        bcol[t] = (long)(n / g.nci) * g.sbo + n % g.nci;
     }
     for (int k0 = 0; k0 < g.K; k0 += 16) {
         bf16x4 ar[3], an[3], ai[3];
@@ -425,7 +519,7 @@ __global__ void __launch_bounds__(256) k_zgemm_bf16x3(ZGemmArgs g) {
         for (int j = 0; j < 4; ++j) {
             const int k = k0 + 4 * q + j;
             const bool va = m < g.M && k < g.K;
-            const long ia = oa + m * g.sam + k * g.sak;
+            const long ia = oa + m * g.sam + k;
             short x0, x1, x2;
             split3(va ? g.Ar[ia] : 0.0, x0, x1, x2);
             ar[0][j] = x0; ar[1][j] = x1; ar[2][j] = x2;
@@ -465,7 +559,7 @@ __global__ void __launch_bounds__(256) k_zgemm_bf16x3(ZGemmArgs g) {
         for (int j = 0; j < 4; ++j) {
             const int row = tm * 16 + 4 * q + j, col = (tg * NT + t) * 16 + r;
             if (row < g.M && col < g.N) {
-                const long ic = oc + row * g.scm + (long)(col / g.nci) * g.sco + (long)(col % g.nci) * g.scn;
+                const long ic = oc + zrow(g, row) + zcol(g, col);
                 g.Cr[ic] = (double)cr[t][j];
                 g.Ci[ic] = (double)ci[t][j];
             }
@@ -474,28 +568,34 @@ __global__ void __launch_bounds__(256) k_zgemm_bf16x3(ZGemmArgs g) {
 
 }  // namespace
 
-int polyeri_zgemm_launch(int mode, int M, int N, int K, const double* Ar, const double* Ai, long sam, long sak,
-                         long sA, const double* Br, const double* Bi, long sbk, long sbn, long sB, double* Cr,
-                         double* Ci, long scm, long scn, long sC, int batch, hipStream_t stream, int nci, long sbo,
-                         long sco) {
+int polyeri_zgemm_launch(int mode, int M, int N, int K, const double* Ar, const double* Ai, long sam, long sA,
+                         const double* Br, const double* Bi, long sbk, long sB, double* Cr, double* Ci, long scm,
+                         long scn, long sC, int batch, hipStream_t stream, int nci, long sbo, long sco, int mci,
+                         long smo) {
     if (M < 1 || N < 1 || K < 1 || batch < 1 || !Ar || !Br || !Bi || !Cr || !Ci) return -1;
     if (nci <= 0) nci = N;
+    if (mci <= 0) mci = M;
     if (mode != GEMM_F64 && mode != GEMM_BF16X3) return -1;
-    // column tiles per wavefront: enough for N (up to 4)
     const int ntile = (N + 15) / 16;
-    const int nt = ntile >= 4 ? 4 : ntile;
+    const int nt = ntile >= 4 ? 4 : ntile;             // BF16x3: column tiles per wavefront
     const long tiles = (long)((M + 15) / 16) * ((N + 16 * nt - 1) / (16 * nt));
     if ((tiles + 3) / 4 > 0x7fffffffL) return -1;
+    // FP64: column tiles per block, fewest padded columns first, then most
+    int tnw = 1;
+    for (int c = 2; c <= 4; ++c)
+        if ((ntile + c - 1) / c * c <= (ntile + tnw - 1) / tnw * tnw) tnw = c;
+    if (ntile > 4 && tnw < 3) tnw = 4;                 // a padded tile costs less than narrow blocks
     for (int b0 = 0; b0 < batch; b0 += 65535) {       // grid.y limit
         const int nb = batch - b0 < 65535 ? batch - b0 : 65535;
-        ZGemmArgs g{M, N, K, Ar + b0 * sA, Ai ? Ai + b0 * sA : nullptr, sam, sak, sA, Br + b0 * sB, Bi + b0 * sB,
-                    sbk, sbn, sB, Cr + b0 * sC, Ci + b0 * sC, scm, scn, sC, nci, sbo, sco};
+        ZGemmArgs g{M, N, K, Ar + b0 * sA, Ai ? Ai + b0 * sA : nullptr, sam, sA, Br + b0 * sB, Bi + b0 * sB,
+                    sbk, sB, Cr + b0 * sC, Ci + b0 * sC, scm, scn, sC, nci, sbo, sco, mci, smo};
         const dim3 grid((unsigned)((tiles + 3) / 4), (unsigned)nb);
         if (mode == GEMM_F64) {
-            if (nt == 1) hipLaunchKernelGGL(k_zgemm_f64<1>, grid, dim3(256), 0, stream, g);
-            else if (nt == 2) hipLaunchKernelGGL(k_zgemm_f64<2>, grid, dim3(256), 0, stream, g);
-            else if (nt == 3) hipLaunchKernelGGL(k_zgemm_f64<3>, grid, dim3(256), 0, stream, g);
-            else hipLaunchKernelGGL(k_zgemm_f64<4>, grid, dim3(256), 0, stream, g);
+            if (tnw == 1 ? launch_zgemm_f64<1>(g, nb, stream)
+                : tnw == 2 ? launch_zgemm_f64<2>(g, nb, stream)
+                : tnw == 3 ? launch_zgemm_f64<3>(g, nb, stream)
+                           : launch_zgemm_f64<4>(g, nb, stream))
+                return -1;
         } else {
             if (nt == 1) hipLaunchKernelGGL(k_zgemm_bf16x3<1>, grid, dim3(256), 0, stream, g);
             else if (nt == 2) hipLaunchKernelGGL(k_zgemm_bf16x3<2>, grid, dim3(256), 0, stream, g);

@@ -1776,6 +1776,58 @@ __global__ void k_fill_u32(unsigned* p, size_t n) {
     if (i < n) p[i] = 0u;
 }
 
+// Independent launches of one call over kBranches streams: the context's own
+// and the device's side streams, which wait for what is enqueued on it so far
+// (fork_branches) and which it waits for afterwards (join_branches).
+static int fork_branches(polyeri_ctx* c) {
+    HIPCHK(hipEventRecord(c->ev_fork, c->stream));
+    for (int i = 0; i < kBranches - 1; ++i) HIPCHK(hipStreamWaitEvent(c->side[i], c->ev_fork, 0));
+    return 0;
+}
+static int join_branches(polyeri_ctx* c) {
+    for (int i = 0; i < kBranches - 1; ++i) {
+        HIPCHK(hipEventRecord(c->ev_join[i], c->side[i]));
+        HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join[i], 0));
+    }
+    return 0;
+}
+// The branch of each of n launches: costliest first, to the least loaded one.
+template <typename Cost>
+static std::vector<int> deal_branches(size_t n, Cost cost) {
+    std::vector<int> branch(n, 0), order(n);
+    for (size_t w = 0; w < n; ++w) order[w] = (int)w;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost(a) > cost(b); });
+    double load[kBranches] = {};
+    for (int w : order) {
+        int bmin = 0;
+        for (int i = 1; i < kBranches; ++i)
+            if (load[i] < load[bmin]) bmin = i;
+        branch[w] = bmin;
+        load[bmin] += cost(w);
+    }
+    return branch;
+}
+// Runs launch(list) for every work list on its branch (all on the context's
+// stream where fork is false); the kernels go to c->stream.
+template <typename Launch>
+static int launch_lists(polyeri_ctx* c, bool fork, Launch launch) {
+    const std::vector<int> branch =
+        fork ? deal_branches(c->work.size(), [&](int w) { return c->work[w].flops; }) : std::vector<int>();
+    int rc = fork ? fork_branches(c) : 0;
+    if (rc) return rc;
+    hipStream_t main = c->stream;
+    for (size_t w = 0; w < c->work.size() && !rc; ++w) {
+        if (fork && branch[w]) c->stream = c->side[branch[w] - 1];
+        rc = launch(w);
+        c->stream = main;
+    }
+    if (fork) {                                   // joined also after a failed launch
+        const int jrc = join_branches(c);
+        if (!rc) rc = jrc;
+    }
+    return rc;
+}
+
 // The kernel sequence of one J/K build of the contracted density d_pc into
 // d_jc / d_kc (reference layout): density packing, zeroing (fill kernels,
 // so the sequence can be captured in a graph), the optional density
@@ -1862,58 +1914,6 @@ static int jk_enqueue(polyeri_ctx* c, const double* d_pc, double* d_jc, double* 
 // One J/K build.  Without per-class profiling the kernel sequence is
 // captured once per (density, J, K, screening) combination into a HIP graph
 // and replayed; the timing events stay outside the graph.
-// Independent launches of one call over kBranches streams: the context's own
-// and the device's side streams, which wait for what is enqueued on it so far
-// (fork_branches) and which it waits for afterwards (join_branches).
-static int fork_branches(polyeri_ctx* c) {
-    HIPCHK(hipEventRecord(c->ev_fork, c->stream));
-    for (int i = 0; i < kBranches - 1; ++i) HIPCHK(hipStreamWaitEvent(c->side[i], c->ev_fork, 0));
-    return 0;
-}
-static int join_branches(polyeri_ctx* c) {
-    for (int i = 0; i < kBranches - 1; ++i) {
-        HIPCHK(hipEventRecord(c->ev_join[i], c->side[i]));
-        HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join[i], 0));
-    }
-    return 0;
-}
-// The branch of each of n launches: costliest first, to the least loaded one.
-template <typename Cost>
-static std::vector<int> deal_branches(size_t n, Cost cost) {
-    std::vector<int> branch(n, 0), order(n);
-    for (size_t w = 0; w < n; ++w) order[w] = (int)w;
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost(a) > cost(b); });
-    double load[kBranches] = {};
-    for (int w : order) {
-        int bmin = 0;
-        for (int i = 1; i < kBranches; ++i)
-            if (load[i] < load[bmin]) bmin = i;
-        branch[w] = bmin;
-        load[bmin] += cost(w);
-    }
-    return branch;
-}
-// Runs launch(list) for every work list on its branch (all on the context's
-// stream where fork is false); the kernels go to c->stream.
-template <typename Launch>
-static int launch_lists(polyeri_ctx* c, bool fork, Launch launch) {
-    const std::vector<int> branch =
-        fork ? deal_branches(c->work.size(), [&](int w) { return c->work[w].flops; }) : std::vector<int>();
-    int rc = fork ? fork_branches(c) : 0;
-    if (rc) return rc;
-    hipStream_t main = c->stream;
-    for (size_t w = 0; w < c->work.size() && !rc; ++w) {
-        if (fork && branch[w]) c->stream = c->side[branch[w] - 1];
-        rc = launch(w);
-        c->stream = main;
-    }
-    if (fork) {                                   // joined also after a failed launch
-        const int jrc = join_branches(c);
-        if (!rc) rc = jrc;
-    }
-    return rc;
-}
-
 // J/K from the stored records (DIRECT .F.) into the reference-layout
 // blocks d_jc / d_kc (ncell blocks: 1 for a molecule).
 static int jk_stored(polyeri_ctx* c, const double* d_pc, double* d_jc, double* d_kc) {
@@ -2203,6 +2203,7 @@ static int tensor_device(polyeri_ctx* c, double* d_t, bool packed = false) {
     int rc = launch_lists(c, true, [&](size_t w) {
         // lists with a generally contracted form of shell-pair groups: one
         // primitive loop per group quartet for all its member quartets
+        const ClassPairWork& cw = c->work[w];
         const bool gc = cw.gc.nwork > 0 && cw.gc.kind == 0;
         return gc ? launch_gc(c, cw, cw.gc_block, nullptr, d_t)
                   : launch_class(c, MODE_TENSOR, cw.la, cw.lb, cw.lc, cw.ld, cw.d_bra, cw.d_ket, cw.d_row, cw.nrows,
@@ -2210,7 +2211,7 @@ static int tensor_device(polyeri_ctx* c, double* d_t, bool packed = false) {
                                  LaunchCfg(), cw.d_bsoa);
     });
     c->tpack = 0;
-    return 0;
+    return rc;
 }
 
 int polyeri_eri_tensor(polyeri_ctx* ctx, double* feri) {
@@ -2283,7 +2284,7 @@ int polyeri_get_stats(polyeri_ctx* ctx, polyeri_stats* st) {
         }
         st->class_l[i] = w.la * 1000 + w.lb * 100 + w.lc * 10 + w.ld;
     }
-    return rc;
+    return 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -2301,7 +2302,6 @@ static void lu_solve(int n, const std::vector<double>& A0, const std::vector<dou
         double m = 0;
         for (int j = 0; j < n; ++j) m = std::max(m, std::fabs(A[i + n * j]));
         sc[i] = m > 0 ? 1.0 / m : 1.0;
-        const ClassPairWork& cw = c->work[w];
     }
     for (int k = 0; k < n; ++k) {
         int p = k;
@@ -3923,7 +3923,7 @@ static int mp2_periodic(polyeri_ctx* ctx, int kvc, const double* co, const doubl
     const long N = n, n1 = 2 * ctx->rc1 + 1, n3 = 2 * ctx->cel2 + 1, NK = nk, NO = nop, NV = nvp;
     const long NB = nvmax;                              // virtual bands of one k_b, at most
     const long M1 = N * n1 * N * n3 * N, M2 = N * n1 * N;
-    if (M1 > INT_MAX || (long)NK * NB * NO > INT_MAX || (long)NB * NO * NV > INT_MAX)
+    if (M1 > INT_MAX || NK * NB * NO * N > INT_MAX || NB * NO * NV > INT_MAX || NB * M2 > INT_MAX)
         return fail(POLYERI_E_ARG, "polyeri_mp2_energy_periodic: lattice tensor too large for one pass");
     const size_t nT = (size_t)M1 * n1 * N;
     const size_t nTN = (size_t)M1 * NB, nTOK = (size_t)NK * NB * NO * M2, nTV = (size_t)NK * NK * NB * NO * NV * N,
@@ -3953,10 +3953,10 @@ static int mp2_periodic(polyeri_ctx* ctx, int kvc, const double* co, const doubl
     double2* dCO;
     int* dPlim;
     int rc;
-    if ((rc = buf.get(&dT, nT)) || (rc = buf.get(&dTNr, nTN)) || (rc = buf.get(&dTNi, nTN)) ||
+    if ((rc = buf.get(&dT, nT)) || (rc = buf.get(&dTNr, kgrp * nTN)) || (rc = buf.get(&dTNi, kgrp * nTN)) ||
         (rc = buf.get(&dTOKr, nTOK)) || (rc = buf.get(&dTOKi, nTOK)) || (rc = buf.get(&dTVr, nTV)) ||
         (rc = buf.get(&dTVi, nTV)) || (rc = buf.get(&dTOVr, nTOV)) || (rc = buf.get(&dTOVi, nTOV)) ||
-        (rc = buf.get(&dB1r, nB1)) || (rc = buf.get(&dB1i, nB1)) || (rc = buf.get(&dB2r, nB2)) ||
+        (rc = buf.get(&dB1r, kgrp * nB1)) || (rc = buf.get(&dB1i, kgrp * nB1)) || (rc = buf.get(&dB2r, nB2)) ||
         (rc = buf.get(&dB2i, nB2)) || (rc = buf.get(&dB3r, nB3)) || (rc = buf.get(&dB3i, nB3)) ||
         (rc = buf.get(&dB4r, nB4)) || (rc = buf.get(&dB4i, nB4)) || (rc = buf.get(&dCr, nC)) ||
         (rc = buf.get(&dCi, nC)) || (rc = buf.get(&dEps, (size_t)nc * nk)) || (rc = buf.get(&dAcc, 2)) ||
@@ -3979,44 +3979,54 @@ static int mp2_periodic(polyeri_ctx* ctx, int kvc, const double* co, const doubl
                        nop, icore, 0, 0, 0, 1, dPlim, dB4r, dB4i);
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, s, dAcc, (size_t)2, 0.0);
     HIPCHK(hipGetLastError());
-    auto gemm = [&](int M, int Nn, int K, const double* Ar, const double* Ai, long sam, long sak, long sA,
-                    const double* Br, const double* Bi, long sbk, long sbn, long sB, double* Cr, double* Ci, long scm,
-                    long scn, long sC, int batch, int nci = 0, long sbo = 0, long sco = 0) {
-        return polyeri_zgemm_launch(mode, M, Nn, K, Ar, Ai, sam, sak, sA, Br, Bi, sbk, sbn, sB, Cr, Ci, scm, scn, sC,
-                                    batch, s, nci, sbo, sco);
+    auto gemm = [&](long M, int Nn, int K, const double* Ar, const double* Ai, long sam, long sA, const double* Br,
+                    const double* Bi, long sbk, long sB, double* Cr, double* Ci, long scm, long scn, long sC,
+                    int batch, int nci = 0, long sbo = 0, long sco = 0, int mci = 0, long smo = 0) {
+        return polyeri_zgemm_launch(mode, (int)M, Nn, K, Ar, Ai, sam, sA, Br, Bi, sbk, sB, Cr, Ci, scm, scn, sC, batch,
+                                    s, nci, sbo, sco, mci, smo);
     };
-    for (int kb = 0; kb < nk; ++kb) {
+    for (int kb = 0, kg = 0; kb < nk; ++kb) {
         const int nb = plim[kb] - iocc;
-        if (nb <= 0) continue;
+        if (nb <= 0) { kg = 0; continue; }
         const long NBk = nb;
-        // Q1 quarter: TN[b][(i,Q1,j,Q3,k)] = sum_{Q2,l} T CO(l,b,kb) e^{i kb Q2} (:253-258;
+        // Q1 quarter: TN[kb][b][(i,Q1,j,Q3,k)] = sum_{Q2,l} T CO(l,b,kb) e^{i kb Q2} (:253-258;
         // the e^{i kb Q3} factor moves into the next operand); b outermost so the
-        // next quarter reads its contraction index (Q3,k) contiguously
-        hipLaunchKernelGGL(k_mp2k_operand, dim3(nblk(nB1)), dim3(256), 0, s, dCr, dCi, nk, n, nc, kvc, kb, 1,
-                           (int)n1, ctx->rc1, nb, iocc, 1, 0, 0, 0, dPlim, dB1r, dB1i);
+        // next quarter reads its contraction index (Q3,k) contiguously.  One product
+        // takes the next kgrp k-points with as many bands, so T is read once for them.
+        if (kg == 0) {
+            while (kg < kgrp && kb + kg < nk && plim[kb + kg] - iocc == nb) ++kg;
+            for (int x = 0; x < kg; ++x)
+                hipLaunchKernelGGL(k_mp2k_operand, dim3(nblk(nB1)), dim3(256), 0, s, dCr, dCi, nk, n, nc, kvc, kb + x,
+                                   1, (int)n1, ctx->rc1, nb, iocc, 1, 0, 0, 0, dPlim, dB1r + x * n1 * N * NBk,
+                                   dB1i + x * n1 * N * NBk);
+            HIPCHK(hipGetLastError());
+            if (gemm(M1, kg * nb, (int)(n1 * N), dT, nullptr, n1 * N, 0, dB1r, dB1i, NBk, 0, dTNr, dTNi, 1, M1, 0, 1,
+                     nb, n1 * N * NBk, NBk * M1))
+                return fail(POLYERI_E_HIP, "k-point MP2: first quarter launch failed");
+            kfirst = kb;
+        }
+        const double *tnr = dTNr + (kb - kfirst) * NBk * M1, *tni = dTNi + (kb - kfirst) * NBk * M1;
+        if (kb - kfirst == kg - 1) kg = 0;
         // B2[kj][(Q3,k)][jo] = conj(CO(k,jo,kj)) e^{i (kb - kj) Q3} (:294-299)
         hipLaunchKernelGGL(k_mp2k_operand, dim3(nblk(nB2)), dim3(256), 0, s, dCr, dCi, nk, n, nc, kvc, 0, nk,
                            (int)n3, ctx->cel2, nop, icore, -1, kb, 1, 1, dPlim, dB2r, dB2i);
         HIPCHK(hipGetLastError());
-        if (gemm((int)M1, nb, (int)(n1 * N), dT, nullptr, n1 * N, 1, 0, dB1r, dB1i, NBk, 1, 0, dTNr, dTNi, 1, M1, 0,
-                 1))
-            return fail(POLYERI_E_HIP, "k-point MP2: first quarter launch failed");
-        // Q2 quarter, every kj in one product (columns (kj, jo)), so TN is
-        // read once: TOK[kj][b][jo][(i,Q1,j)] = sum_{Q3,k} TN B2[kj]
-        if (gemm((int)M2, nk * nop, (int)(n3 * N), dTNr, dTNi, n3 * N, 1, M1, dB2r, dB2i, NO, 1, 0, dTOKr, dTOKi, 1,
-                 M2, NO * M2, nb, nop, n3 * N * NO, NBk * NO * M2))
+        // Q2 quarter, every b (rows) and kj (columns (kj, jo)) in one product, so
+        // TN is read once: TOK[kj][b][jo][(i,Q1,j)] = sum_{Q3,k} TN B2[kj]
+        if (gemm(NBk * M2, nk * nop, (int)(n3 * N), tnr, tni, n3 * N, 0, dB2r, dB2i, NO, 0, dTOKr, dTOKi, 1, M2, 0, 1,
+                 nop, n3 * N * NO, NBk * NO * M2, (int)M2, NO * M2))
             return fail(POLYERI_E_HIP, "k-point MP2: second quarter launch failed");
-        // Q3 quarter, every ka in one product (columns (ka, a)):
+        // Q3 quarter, every (kj, b, jo) (rows) and ka (columns (ka, a)) in one product:
         // TV[ka][(kj,b,jo)][a][i] = sum_{Q1,j} TOK B3[ka]
-        if (gemm((int)N, nk * nvp, (int)(n1 * N), dTOKr, dTOKi, n1 * N, 1, M2, dB3r, dB3i, NV, 1, 0, dTVr, dTVi, 1,
-                 N, NV * N, nk * nb * nop, nvp, n1 * N * NV, NK * NBk * NO * NV * N))
+        if (gemm(NK * NBk * NO * N, nk * nvp, (int)(n1 * N), dTOKr, dTOKi, n1 * N, 0, dB3r, dB3i, NV, 0, dTVr, dTVi, 1,
+                 N, 0, 1, nvp, n1 * N * NV, NK * NBk * NO * NV * N, (int)N, NV * N))
             return fail(POLYERI_E_HIP, "k-point MP2: third quarter launch failed");
         // Q4 quarter, per kj, batched over ka with ki = ka + (kb - kj mod nk):
         // TOV[kj][ka][(b,jo,a)][io] = sum_i TV[ka][kj] conj(CO(i,io,ki))
         for (int kj = 0; kj < nk; ++kj) {
             const long d = ((kb - kj) % nk + nk) % nk;
-            if (gemm(nb * nop * nvp, nop, (int)N, dTVr + kj * NBk * NO * NV * N, dTVi + kj * NBk * NO * NV * N, N, 1,
-                     NK * NBk * NO * NV * N, dB4r + d * N * NO, dB4i + d * N * NO, NO, 1, N * NO,
+            if (gemm((long)nb * nop * nvp, nop, (int)N, dTVr + kj * NBk * NO * NV * N, dTVi + kj * NBk * NO * NV * N, N,
+                     NK * NBk * NO * NV * N, dB4r + d * N * NO, dB4i + d * N * NO, NO, N * NO,
                      dTOVr + kj * NK * NBk * NO * NV * NO, dTOVi + kj * NK * NBk * NO * NV * NO, NO, 1,
                      NBk * NO * NV * NO, nk))
                 return fail(POLYERI_E_HIP, "k-point MP2: fourth quarter launch failed");
