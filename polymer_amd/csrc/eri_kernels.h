@@ -24,8 +24,8 @@ struct PairMeta {
 
 // A segment of one bra row: items t0 .. t0 + n - 1 of the list, all with
 // the bra pair of row `row`.  2^ls lanes of a wavefront share each item and
-// divide its ket primitive pairs (k_eri_seg, k_eri_gc, k_eri_gck; ls = 0 in
-// the lists of the other kernels).
+// divide its ket primitive pairs (k_eri_seg, k_eri_gc, k_eri_gck; in the Rys
+// classes k_eri_rys, 2^ls groups of a member's lanes).
 struct SegDesc {
     long long t0;
     int row;

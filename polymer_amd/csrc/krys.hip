@@ -87,7 +87,12 @@ POLY_HD void rys_prim(const PrimPair& bq, double PA0, double PA1, double PA2, co
 }
 
 // One variant of the class over the items of one segment that this wave
-// owns: chunk c of the segment's items goes to wave (c + base) % nw.  MODE:
+// owns: chunk c of the segment's items goes to wave (c + base) % nw.  The ket
+// primitive pairs of an item are divided over 2^ls groups of NMEMB lanes (the
+// segment's ls, as many groups as a wavefront holds) and the groups' integrals
+// summed before the digestion: in a small molecule, where one group did 64
+// primitive quartets of three roots one after the other, that chain was the
+// whole launch (one water cc-pVDZ, (dp|pp): 165 us, divided 34 us).  MODE:
 // MODE_JK (FP64) or MODE_JK32 (recursion and per-lane integrals in FP32;
 // nodes, weights, pair data and the digestion in FP64).
 template <int LA, int LB, int LC, int LD, int V, int MODE>
@@ -99,10 +104,11 @@ __device__ __forceinline__ void rys_variant(const EriArgs& g, const SegDesc& seg
     using real = typename std::conditional<MODE == MODE_JK32, float, double>::type;
     constexpr int NA = ncart(LA), NB = ncart(LB);
     const int lane = threadIdx.x & 63;
-    constexpr int IPW = 64 / R::NMEMB;
+    const int lp = min((int)seg.ls, R::NMEMB > 4 ? 3 : 4);   // 2^lp lanes a member
+    const int IPW = (64 / R::NMEMB) >> lp;
     const int chunks = (seg.n + IPW - 1) / IPW;
     const int n = g.nbf;
-    const int memb = lane % R::NMEMB, slot = lane / R::NMEMB;
+    const int memb = lane % R::NMEMB, part = (lane / R::NMEMB) & ((1 << lp) - 1), slot = lane / R::NMEMB >> lp;
     int p[3];
     R::perm(memb, p[0], p[1], p[2]);
     int gA[R::NA], gB[R::NB], gC[R::NC], gD[R::ND];
@@ -137,8 +143,8 @@ __device__ __forceinline__ void rys_variant(const EriArgs& g, const SegDesc& seg
                 live = g.Qs[bp] * g.Qs[kp] * m >= g.dtol;
             }
         }
-        if (screen) {   // one count per item (member 0)
-            const unsigned long long mask = __ballot(live && memb == 0);
+        if (screen) {   // one count per item (member 0, part 0)
+            const unsigned long long mask = __ballot(live && memb == 0 && part == 0);
             if (lane == 0 && mask) atomicAdd(g.kept, (unsigned)__popcll(mask));
         }
         if (!live) continue;
@@ -155,10 +161,14 @@ __device__ __forceinline__ void rys_variant(const EriArgs& g, const SegDesc& seg
             const PrimPair bq = scalar_load(bra + pi);
             const double PAg[3] = {bq.PAx, bq.PAy, bq.PAz};
             const double PA0 = sel3(PAg, p[0]), PA1 = sel3(PAg, p[1]), PA2 = sel3(PAg, p[2]);
-            for (int qi = 0; qi < mk.nprim; ++qi)
+            for (int qi = part; qi < mk.nprim; qi += 1 << lp)
                 rys_prim<R, real>(bq, PA0, PA1, PA2, kv.load(qi), p, ABl0, ABl1, ABl2, CDl0, CDl1, CDl2,
                                   rys_tab<R::NROOT>(), rys_herm<R::NROOT>(), accr);
         }
+        for (int st = 1 << lp >> 1; st; st >>= 1)   // parts are NMEMB lanes apart; part 0 ends with the sums
+#pragma unroll
+            for (int i = 0; i < R::NOUT; ++i) accr[i] += __shfl(accr[i], lane + st * R::NMEMB);
+        if (part) continue;
         // digestion of the lane's integrals v(a, b, c, d) (local components)
         const double s = (fa == fb ? 0.5 : 1.0) * (fc == fd ? 0.5 : 1.0) * (bp == kp ? 0.5 : 1.0);
         const double* D = g.D;

@@ -278,9 +278,11 @@ static double flop_model(int la, int lb, int lc, int ld) {
 enum { LAUNCH_AUTO = 0, LAUNCH_REG = 1, LAUNCH_COOP = 2, LAUNCH_SEG = 3, LAUNCH_RYS = 5 };
 static const int RYS_NMAX_EXPORT = 5;
 // Items per bra-row segment of the segment kernel (at most), and the number
-// of segments a list's primitive quartets are spread over (at least).
+// of segments a list's primitive quartets are spread over (at least); the
+// Rys classes' segments and least items (make_segments).
 static const int kSegItems = 2048, kSegMin = 256;
 static const double kSegTarget = 4096.0;
+static const long long kSegTargetRys = 1024, kSegMinRys = 16;
 
 // Lanes (log2) that share one item of bp bra and kp ket primitive pairs.  One
 // lane per item makes the longest chain of a deeply contracted basis, 81 x 81
@@ -295,11 +297,11 @@ static const double kSegTarget = 4096.0;
 // about one digestion's time to several).  In a large build only the longest
 // items are shared, in a small one, whose lanes are idle, nearly all.
 static const double kSplitLanes = 256.0 * 4 * 64 * 2, kSplitMin = 8.0, kSplitMax = 128.0;
-static int segment_split(double bp, double kp, double list_total, double ctx_total) {
+static int segment_split(double bp, double kp, double list_total, double ctx_total, int lsmax) {
     const double limit = std::max(0.5 * list_total / kSplitLanes,
                                   std::min(std::max(ctx_total / kSplitLanes / 16.0, kSplitMin), kSplitMax));
     int ls = 0;
-    while (ls < 6 && (1 << ls) < kp && bp * kp > limit * (1 << ls)) ++ls;
+    while (ls < lsmax && (1 << ls) < kp && bp * kp > limit * (1 << ls)) ++ls;
     return ls;
 }
 
@@ -315,14 +317,22 @@ static int segment_split(double bp, double kp, double list_total, double ctx_tot
 // each), so a row is also cut where that changes.  pairs / bra / kets /
 // bstart: the list's pair data, bra ids by row, ket ids and bucket starts of
 // the ket class.  balanced = false: rows cut every kSegItems lanes, in row
-// order (the autotuner keeps whichever form is faster per list).
+// order (the autotuner keeps whichever form is faster per list).  rys: the
+// list of a Rys class, whose items take 3 or 6 lanes of each of 1 to 8
+// variants (so up to 2^4 groups of lanes may share one) and far outweigh a
+// row flush: short lists are cut finer, into about kSegTargetRys segments of
+// at least kSegMinRys items, four blocks a CU ((H2O)16 cc-pVDZ, 103 -> 1092
+// segments of (dd|dp): 0.31 -> 0.15 ms; lists of 1000 segments and more lose
+// to the flushes, (dp|pp) of 2066 -> 3599: 0.67 -> 0.74 ms, and stay).
 static std::vector<SegDesc> make_segments(const WorkList& l, const std::vector<PairInfo>& pairs,
                                           const std::vector<int>& bra, const std::vector<int>& kets,
-                                          const std::vector<int>& bstart, double split, bool balanced = true) {
+                                          const std::vector<int>& bstart, double split, bool balanced = true,
+                                          bool rys = false) {
     const int nb = l.nbucket;
     std::vector<double> knp(nb, 0.0);
     for (int b = 0; b + 1 < (int)bstart.size() && b < nb; ++b) knp[b] = pairs[kets[bstart[b]]].nprim;
     const double target = balanced ? l.prim_quartets / kSegTarget : 1e300;
+    const int least = rys ? (int)std::clamp<long long>(l.nwork / kSegTargetRys, kSegMinRys, kSegMin) : kSegMin;
     std::vector<std::pair<double, SegDesc>> segs;
     for (int r = 0; r < l.nrows; ++r) {
         const double bp = pairs[bra[r]].nprim;
@@ -338,10 +348,10 @@ static std::vector<SegDesc> make_segments(const WorkList& l, const std::vector<P
             int cnt = rb[b + 1] - rb[b];
             if (cnt <= 0) continue;
             const double ci = bp * knp[b];
-            const int lb = split > 0.0 ? segment_split(bp, knp[b], l.prim_quartets, split) : 0;
+            const int lb = split > 0.0 ? segment_split(bp, knp[b], l.prim_quartets, split, rys ? 4 : 6) : 0;
             if (lb != ls) flush();
             ls = lb;
-            const int nmax = kSegItems >> ls, nmin = kSegMin >> ls;
+            const int nmax = kSegItems >> ls, nmin = std::max(1, least >> ls);
             while (cnt > 0) {
                 int take = std::min(cnt, nmax - n);
                 if (ci > 0.0)
@@ -1389,12 +1399,11 @@ static int build_ctx(polyeri_ctx* c) {
         // stays in bounds), so it is not launched, and mixed contexts do not
         // split the light classes.
         if (!c->pbc && l.nwork > 0 && (!l.prec || polyeri_rys_class(w.la, w.lb, w.lc, w.ld))) {
-            // the Rys kernel has its own lanes per item
-            const double split = polyeri_rys_class(w.la, w.lb, w.lc, w.ld) ? 0.0 : all;
+            const bool rys = polyeri_rys_class(w.la, w.lb, w.lc, w.ld);
             std::vector<SegDesc> segs =
-                make_segments(l, c->pairs, c->class_ids[l.X], c->ket_ids[l.Y], c->bstart[l.Y], split);
+                make_segments(l, c->pairs, c->class_ids[l.X], c->ket_ids[l.Y], c->bstart[l.Y], all, true, rys);
             const std::vector<SegDesc> segc =
-                make_segments(l, c->pairs, c->class_ids[l.X], c->ket_ids[l.Y], c->bstart[l.Y], split, false);
+                make_segments(l, c->pairs, c->class_ids[l.X], c->ket_ids[l.Y], c->bstart[l.Y], all, false, rys);
             if (segs.size() + segc.size() > 0x7fffffffu) return fail(POLYERI_E_ARG, "too many segments");
             w.nseg = (int)segs.size();
             w.nsegc = (int)segc.size();

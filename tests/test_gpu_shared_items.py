@@ -78,3 +78,55 @@ def test_boys_rows_outside_lds_match_register_kernels():
     jr, kr = ctx.fourindex_eri(p)
     assert np.max(np.abs(jr)) > 1
     assert np.max(np.abs(j - jr)) < 2.4e-10 and np.max(np.abs(k - kr)) < 2.4e-10
+
+
+# p of six and d of two primitives: 36 ket primitive pairs in (pp|, 144 and
+# more primitive quartets an item, the most lanes a Rys item can be given
+DEEP_BASIS = """****
+{el}     0
+S    1   1.00
+      6.0000000E-01          1.0000000
+P    6   1.00
+      9.5000000E+00          2.0000000E-02
+      4.1000000E+00          9.0000000E-02
+      2.0000000E+00          2.2000000E-01
+      1.0500000E+00          3.5000000E-01
+      5.5000000E-01          3.3000000E-01
+      2.9000000E-01          1.5000000E-01
+D    2   1.00
+      1.7000000E+00          4.0000000E-01
+      6.3000000E-01          7.0000000E-01
+****
+"""
+
+
+@pytest.mark.parametrize("atoms", [[(10, 0.1, 0.0, -0.2)], [(10, 0.0, 0.1, 0.0), (10, 0.3, -0.2, 2.2)]],
+                         ids=["one_centre", "two_centres"])
+def test_shared_rys_items_match_oracle(tmp_path, atoms):
+    """The Rys classes with 8 (six-lane members) and 16 (three-lane members)
+    lane groups an item, against the oracle and with the screen that keeps
+    every quartet; and the mixed-precision lists.  Tolerance as above; FP32
+    lists: integrals below the cut 1 times 2^-24 per operation of a sum of at
+    most 10^3 terms an element, 1e-3 of the largest element."""
+    path = str(tmp_path / "deep")
+    with open(path, "w") as f:
+        f.write(DEEP_BASIS.format(el="Ne"))
+    b = pa.read_basis(path, atoms)
+    rng = np.random.default_rng(5)
+    real = b.real_functions
+    p = np.zeros((b.ncgs, b.ncgs))
+    a = 0.1 * rng.standard_normal((len(real), len(real)))
+    p[np.ix_(real, real)] = a + a.T
+    ctx = pa.Context(b, schwarz_tol=0.0)
+    print(f"case: shared Rys items, {len(atoms)} centres", flush=True)
+    j, k = ctx.fourindex_eri(p)
+    assert any(c["kernel"] == "rys" and c["quartets"] for c in ctx.stats()["classes"])
+    jr, kr = oracle.Basis(path, atoms).fourindex_eri(p, 0.0)[:2]
+    assert np.max(np.abs(jr)) > 0 and np.max(np.abs(kr)) > 0
+    assert np.max(np.abs(j - jr)) < 1e-10 and np.max(np.abs(k - kr)) < 1e-10
+    js, ks = ctx.fourindex_eri(p, dens_tol=1e-290)
+    assert np.max(np.abs(js - jr)) < 1e-10 and np.max(np.abs(ks - kr)) < 1e-10
+    mixed = pa.Context(b, schwarz_tol=0.0, precision=pa.MIXED, mixed_cut=1.0)
+    jm, km = mixed.fourindex_eri(p)
+    assert np.max(np.abs(jm - jr)) < 1e-3 * np.max(np.abs(jr))
+    assert np.max(np.abs(km - kr)) < 1e-3 * np.max(np.abs(kr))
