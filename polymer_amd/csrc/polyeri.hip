@@ -58,6 +58,7 @@ int polyeri_record_error(int code, const char* msg) { return fail(code, msg ? ms
 // ---------------------------------------------------------------------------
 #include "eri_kernels.h"
 #include "kcc.h"
+#include "work_pool.h"
 
 __global__ void k_fill(double* p, size_t n, double v) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -597,105 +598,37 @@ static int ensure_onee_device(polyeri_ctx* c) {
     return 0;
 }
 
-// Work buffers of single calls (MP2, CC, gradient, k-point SCF), kept between
-// calls: mapping and unmapping gigabytes on each call took longer than the
-// call ((H2O)8 cc-pVDZ MP2: 17 ms of kernels, 130 to 270 ms with hipMalloc and
-// hipFree of its 9 GB in a process that holds other allocations).  A block is
-// handed out only while it is in use by nobody (mutex; the caller waits for
-// its streams before it gives a block back).  At most a quarter of the
-// device's memory is kept idle, all of it goes back when the device's last
-// context ends or an allocation fails.
-struct WorkPool {
-    struct Block {
-        void* p;
-        size_t bytes;
-        int device;
-    };
-    std::mutex mu;
-    std::vector<Block> idle, used;
-    std::vector<int> contexts;            // live contexts per device
-
-    size_t idle_bytes(int device) {
+// The device's allocator under the work pool.
+struct HipMemory {
+    static int device() {
+        int d = 0;
+        const hipError_t e = hipGetDevice(&d);
+        return e == hipSuccess ? d : -(int)e;
+    }
+    static int alloc(void** p, size_t bytes) {
+        const hipError_t e = hipMalloc(p, bytes);
+        if (e != hipSuccess) (void)hipGetLastError();
+        return (int)e;
+    }
+    static void free(void* p) { (void)hipFree(p); }
+    static size_t total(int device) {
         size_t n = 0;
-        for (const Block& b : idle) n += b.device == device ? b.bytes : 0;
-        return n;
-    }
-    void release(int device) {            // with mu held
-        for (size_t i = idle.size(); i-- > 0;)
-            if (idle[i].device == device) {
-                (void)hipFree(idle[i].p);
-                idle.erase(idle.begin() + i);
-            }
-    }
-    hipError_t get(void** p, size_t bytes) {
-        int device = 0;
-        hipError_t e = hipGetDevice(&device);
-        if (e != hipSuccess) return e;
-        std::lock_guard<std::mutex> lk(mu);
-        size_t best = idle.size();        // the smallest idle block that holds it and is not twice too large
-        for (size_t i = 0; i < idle.size(); ++i)
-            if (idle[i].device == device && idle[i].bytes >= bytes && idle[i].bytes / 2 <= bytes + 32768 &&
-                (best == idle.size() || idle[i].bytes < idle[best].bytes))
-                best = i;
-        if (best < idle.size()) {
-            used.push_back(idle[best]);
-            idle.erase(idle.begin() + best);
-        } else {
-            void* q = nullptr;
-            e = hipMalloc(&q, bytes);
-            if (e != hipSuccess) {
-                (void)hipGetLastError();
-                release(device);
-                e = hipMalloc(&q, bytes);
-            }
-            if (e != hipSuccess) return e;
-            used.push_back({q, bytes, device});
-        }
-        *p = used.back().p;
-        return hipSuccess;
-    }
-    void put(void* p) {
-        std::lock_guard<std::mutex> lk(mu);
-        for (size_t i = 0; i < used.size(); ++i) {
-            if (used[i].p != p) continue;
-            const Block b = used[i];
-            used.erase(used.begin() + i);
-            size_t freeb = 0, total = 0;
-            if (hipMemGetInfo(&freeb, &total) == hipSuccess && idle_bytes(b.device) + b.bytes <= total / 4)
-                idle.push_back(b);
-            else
-                (void)hipFree(b.p);
-            return;
-        }
-    }
-    void context(int device, int step) {
-        std::lock_guard<std::mutex> lk(mu);
-        if ((int)contexts.size() <= device) contexts.resize(device + 1, 0);
-        contexts[device] += step;
-        if (contexts[device] <= 0) release(device);
+        return hipDeviceTotalMem(&n, device) == hipSuccess ? n : 0;
     }
 };
+using DevicePool = WorkPool<HipMemory>;
 // never destroyed: a context may end after the static objects
-static WorkPool& work_pool() {
-    static WorkPool* pool = new WorkPool;
+static DevicePool& work_pool() {
+    static DevicePool* pool = new DevicePool;
     return *pool;
 }
-int polyeri_work_get(void** p, size_t bytes) { return work_pool().get(p, bytes) == hipSuccess ? 0 : -1; }
+int polyeri_work_get(void** p, size_t bytes) { return work_pool().get(p, bytes); }
 void polyeri_work_put(void* p) { work_pool().put(p); }
 
 template <typename T>
 static int dalloc(T** p, size_t n) {
     if (n == 0) n = 1;
-    hipError_t e = hipMalloc((void**)p, n * sizeof(T));
-    if (e != hipSuccess) {                // idle work buffers may be in the way
-        (void)hipGetLastError();
-        int device = 0;
-        if (hipGetDevice(&device) == hipSuccess) {
-            std::lock_guard<std::mutex> lk(work_pool().mu);
-            work_pool().release(device);
-        }
-        e = hipMalloc((void**)p, n * sizeof(T));
-    }
+    const hipError_t e = (hipError_t)work_pool().alloc((void**)p, n * sizeof(T));
     if (e != hipSuccess) return fail(POLYERI_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     return 0;
 }
@@ -2392,7 +2325,7 @@ struct DevBuf {
     template <typename T>
     int get(T** p, size_t n) {
         void* q = nullptr;
-        const hipError_t e = work_pool().get(&q, std::max<size_t>(n, 1) * sizeof(T));
+        const hipError_t e = (hipError_t)work_pool().get(&q, std::max<size_t>(n, 1) * sizeof(T));
         if (e != hipSuccess) return fail(POLYERI_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
         ptrs.push_back(q);
         *p = static_cast<T*>(q);
@@ -3943,10 +3876,7 @@ static int mp2_periodic(polyeri_ctx* ctx, int kvc, const double* co, const doubl
                         sizeof(double2) * (size_t)nc * nc * nk;
     size_t freeb = 0, totalb = 0;
     HIPCHK(hipMemGetInfo(&freeb, &totalb));
-    {
-        std::lock_guard<std::mutex> lk(work_pool().mu);   // idle work buffers are reused or released
-        freeb += work_pool().idle_bytes(ctx->device);
-    }
+    freeb += work_pool().idle_bytes(ctx->device);     // reused or released
     if (need > freeb - freeb / 16)
         return fail(POLYERI_E_NOMEM, "polyeri_mp2_energy_periodic: " + std::to_string(need >> 20) +
                                          " MiB of transform buffers exceed free device memory");
