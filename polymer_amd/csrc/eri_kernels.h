@@ -1436,10 +1436,6 @@ int polyeri_zgemm_launch(int mode, int M, int N, int K, const double* Ar, const 
                          const double* Br, const double* Bi, long sbk, long sB, double* Cr, double* Ci, long scm,
                          long scn, long sC, int batch, hipStream_t stream, int nci = 0, long sbo = 0, long sco = 0,
                          int mci = 0, long smo = 0);
-// Work buffers kept between calls (polyeri.hip, WorkPool): a block of the
-// current device, and its return once no stream uses it.
-int polyeri_work_get(void** p, size_t bytes);
-void polyeri_work_put(void* p);
 // Density screening (kscreen.hip): shell-block maxima of |D|, and the
 // compaction of one work list to the items whose bound
 // Q_ab Q_cd max(|D| over the six blocks the quartet reads) reaches tol.

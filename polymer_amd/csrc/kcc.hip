@@ -27,6 +27,7 @@
 #include <string>
 #include <vector>
 
+#include "device_memory.h"
 #include "eri_kernels.h"
 
 namespace {

@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/polyeri.h"
+#include "device_memory.h"
 
 // polyeri.hip: records the message returned by polyeri_last_error()
 int polyeri_record_error(int code, const char* msg);
@@ -181,10 +182,10 @@ static int ensure_batch(polyeri_mlp* m, int batch) {
     m->d_z.assign(m->nl + 1, nullptr);
     m->d_a.assign(m->nl + 1, nullptr);
     for (int l = 1; l <= m->nl; ++l) {
-        MCHK(hipMalloc((void**)&m->d_z[l], sizeof(float) * (size_t)batch * m->dim[l]));
-        MCHK(hipMalloc((void**)&m->d_a[l], sizeof(float) * (size_t)batch * m->dim[l]));
+        MCHK(polyeri_device_malloc((void**)&m->d_z[l], sizeof(float) * (size_t)batch * m->dim[l]));
+        MCHK(polyeri_device_malloc((void**)&m->d_a[l], sizeof(float) * (size_t)batch * m->dim[l]));
     }
-    MCHK(hipMalloc((void**)&m->d_part, sizeof(float) * (size_t)nb((long)batch * m->dim[m->nl])));
+    MCHK(polyeri_device_malloc((void**)&m->d_part, sizeof(float) * (size_t)nb((long)batch * m->dim[m->nl])));
     m->cap = batch;
     return 0;
 }
@@ -223,10 +224,10 @@ int polyeri_mlp_create(int nlayers, const int* dims, unsigned long long seed, po
         for (long i = 0; i < (long)dims[l] * dims[l - 1]; ++i) p[m->woff[l - 1] + i] = (float)((2.0 * uni() - 1.0) * sc);
     }
     int rc = 0;
-    hipError_t e = hipMalloc((void**)&m->d_p, sizeof(float) * m->nparam);
-    if (e == hipSuccess) e = hipMalloc((void**)&m->d_g, sizeof(float) * m->nparam);
-    if (e == hipSuccess) e = hipMalloc((void**)&m->d_m1, sizeof(float) * m->nparam);
-    if (e == hipSuccess) e = hipMalloc((void**)&m->d_m2, sizeof(float) * m->nparam);
+    hipError_t e = polyeri_device_malloc((void**)&m->d_p, sizeof(float) * m->nparam);
+    if (e == hipSuccess) e = polyeri_device_malloc((void**)&m->d_g, sizeof(float) * m->nparam);
+    if (e == hipSuccess) e = polyeri_device_malloc((void**)&m->d_m1, sizeof(float) * m->nparam);
+    if (e == hipSuccess) e = polyeri_device_malloc((void**)&m->d_m2, sizeof(float) * m->nparam);
     if (e == hipSuccess) e = hipMemcpy(m->d_p, p.data(), sizeof(float) * m->nparam, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemset(m->d_m1, 0, sizeof(float) * m->nparam);
     if (e == hipSuccess) e = hipMemset(m->d_m2, 0, sizeof(float) * m->nparam);

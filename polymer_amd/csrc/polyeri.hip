@@ -47,9 +47,12 @@ int polyeri_record_error(int code, const char* msg) { return fail(code, msg ? ms
                         std::string(#x) + ": " + hipGetErrorString(e_));                 \
     } while (0)
 
+// A call that found no memory for its workspace (it has not started then) is
+// made again without the idle work buffers.
 #define RBCHK(x)                                                                         \
     do {                                                                                 \
         int s_ = (int)(x);                                                               \
+        if (s_ == rocblas_status_memory_error && release_idle_work()) s_ = (int)(x);     \
         if (s_ != 0) return fail(POLYERI_E_LIB, std::string(#x) + " failed, status " + std::to_string(s_)); \
     } while (0)
 
@@ -57,6 +60,7 @@ int polyeri_record_error(int code, const char* msg) { return fail(code, msg ? ms
 // Kernels
 // ---------------------------------------------------------------------------
 #include "eri_kernels.h"
+#include "device_memory.h"
 #include "kcc.h"
 #include "work_pool.h"
 
@@ -588,16 +592,6 @@ static void drop_graphs(polyeri_ctx* c) {
     c->graphs.clear();
 }
 
-static int ensure_onee_device(polyeri_ctx* c) {
-    if (c->d_T) return 0;
-    size_t n2 = c->T_C.size();
-    HIPCHK(hipMalloc((void**)&c->d_T, n2 * sizeof(double)));
-    HIPCHK(hipMalloc((void**)&c->d_V, n2 * sizeof(double)));
-    HIPCHK(hipMemcpy(c->d_T, c->T_C.data(), n2 * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->d_V, c->N_C.data(), n2 * sizeof(double), hipMemcpyHostToDevice));
-    return 0;
-}
-
 // The device's allocator under the work pool.
 struct HipMemory {
     static int device() {
@@ -622,14 +616,31 @@ static DevicePool& work_pool() {
     static DevicePool* pool = new DevicePool;
     return *pool;
 }
+hipError_t polyeri_device_malloc(void** p, size_t bytes) { return (hipError_t)work_pool().alloc(p, bytes); }
 int polyeri_work_get(void** p, size_t bytes) { return work_pool().get(p, bytes); }
 void polyeri_work_put(void* p) { work_pool().put(p); }
+
+// Gives the current device's idle work buffers back; false where there are none.
+static bool release_idle_work() {
+    const int device = HipMemory::device();
+    return device >= 0 && work_pool().release(device) > 0;
+}
 
 template <typename T>
 static int dalloc(T** p, size_t n) {
     if (n == 0) n = 1;
-    const hipError_t e = (hipError_t)work_pool().alloc((void**)p, n * sizeof(T));
+    const hipError_t e = polyeri_device_malloc((void**)p, n * sizeof(T));
     if (e != hipSuccess) return fail(POLYERI_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    return 0;
+}
+
+static int ensure_onee_device(polyeri_ctx* c) {
+    if (c->d_T) return 0;
+    size_t n2 = c->T_C.size();
+    int rc;
+    if ((rc = dalloc(&c->d_T, n2)) || (rc = dalloc(&c->d_V, n2))) return rc;
+    HIPCHK(hipMemcpy(c->d_T, c->T_C.data(), n2 * sizeof(double), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(c->d_V, c->N_C.data(), n2 * sizeof(double), hipMemcpyHostToDevice));
     return 0;
 }
 
@@ -2072,7 +2083,7 @@ int polyeri_jk_build_screened(polyeri_ctx* ctx, const double* p_c, double dens_t
 int polyeri_device_alloc(polyeri_ctx* ctx, size_t bytes, void** ptr) {
     if (!ctx || !ptr) return fail(POLYERI_E_ARG, "polyeri_device_alloc: null argument");
     HIPCHK(hipSetDevice(ctx->device));
-    HIPCHK(hipMalloc(ptr, bytes ? bytes : 1));
+    HIPCHK(polyeri_device_malloc(ptr, bytes ? bytes : 1));
     return 0;
 }
 
@@ -2344,7 +2355,7 @@ int ScfArena::get_bytes(void** p, size_t bytes) {
         return 0;
     }
     void* q = nullptr;
-    hipError_t e = hipMalloc(&q, bytes);
+    hipError_t e = polyeri_device_malloc(&q, bytes);
     if (e != hipSuccess) return fail(POLYERI_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     if (next < bufs.size()) {
         (void)hipFree(bufs[next].first);

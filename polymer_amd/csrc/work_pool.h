@@ -15,8 +15,8 @@ namespace polyeri {
 // its streams before it gives a block back), and only for a request of nearly
 // its size, so that a call never holds noticeably more than it asked for.  At
 // most a quarter of a device's memory is kept idle; all of a device's idle
-// blocks go back when its last context ends and when an allocation through
-// get or alloc fails.
+// blocks go back when its last context ends and when an allocation of the
+// library fails (get, alloc; release for those that rocBLAS and rocSOLVER make).
 //
 // Mem: the device's allocator, with static functions
 //   int device()                     the current device, negative on error
@@ -107,6 +107,11 @@ class WorkPool {
         std::lock_guard<std::mutex> lk(mu);
         drop(device);                     // another thread may have done so: tried again all the same
         return Mem::alloc(p, bytes);
+    }
+    // Gives a device's idle blocks back; their bytes.
+    size_t release(int device) {
+        std::lock_guard<std::mutex> lk(mu);
+        return drop(device);
     }
     size_t idle_bytes(int device) {
         std::lock_guard<std::mutex> lk(mu);

@@ -2,7 +2,9 @@
 device's allocator: two devices of a few megabytes whose allocations fail where
 their memory ends, as a device's do.  The header is compiled with g++; no GPU."""
 import ctypes
+import glob
 import os
+import re
 import subprocess
 
 import pytest
@@ -53,6 +55,7 @@ void* get(size_t n) { void* p = nullptr; return pool->get(&p, n) ? nullptr : p; 
 void put(void* p) { pool->put(p); }
 void* raw(size_t n) { void* p = nullptr; return pool->alloc(&p, n) ? nullptr : p; }
 size_t size_of(void* p) { return Fake::blocks[p].first; }
+size_t release(int d) { return pool->release(d); }
 void context(int d, int step) { pool->context(d, step); }
 }
 """
@@ -71,7 +74,7 @@ def shim(tmp_path_factory):
     p, n, i = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int
     for name, res, args in [("start", None, [n, n]), ("set_device", None, [i]), ("in_use", n, [i]), ("idle", n, [i]),
                             ("get", p, [n]), ("put", None, [p]), ("raw", p, [n]), ("size_of", n, [p]),
-                            ("context", None, [i, i])]:
+                            ("context", None, [i, i]), ("release", n, [i])]:
         getattr(L, name).restype, getattr(L, name).argtypes = res, args
     return L
 
@@ -142,3 +145,26 @@ def test_failed_allocation_reclaims_idle_blocks(shim):
         assert request(90 * MB)
         assert shim.idle(0) == 0 and shim.idle(1) == 20 * MB
         assert not request(11 * MB)                         # really full
+
+
+def test_release_gives_back_one_devices_idle_blocks(shim):
+    shim.start(100 * MB, 100 * MB)
+    p, q = shim.get(5 * MB), shim.get(6 * MB)
+    shim.put(p)
+    assert shim.release(1) == 0 and shim.release(0) == 5 * MB and shim.release(0) == 0
+    assert shim.in_use(0) == 6 * MB                         # the block in use stays
+    shim.put(q)
+    assert shim.idle(0) == 6 * MB
+
+
+def test_every_allocation_of_the_library_reclaims():
+    """hipMalloc is called in one place, under the pool; every other device
+    allocation goes through the functions that reclaim idle blocks."""
+    csrc = os.path.join(ROOT, "polymer_amd", "csrc")
+    calls = []
+    for path in glob.glob(os.path.join(csrc, "**", "*"), recursive=True):
+        if path.endswith((".hip", ".cpp", ".h")) and "_build" not in path:
+            for line in open(path):
+                if re.search(r"\bhip(Ext)?Malloc\w*\s*\(", line.split("//")[0]) and '"hipMalloc' not in line:
+                    calls.append((os.path.basename(path), line.strip()))
+    assert calls == [("polyeri.hip", "const hipError_t e = hipMalloc(p, bytes);")]
