@@ -117,6 +117,13 @@ int polyeri_sync(polyeri_ctx *ctx);
 int polyeri_device_alloc(polyeri_ctx *ctx, size_t bytes, void **ptr);
 int polyeri_device_free(polyeri_ctx *ctx, void *ptr);
 int polyeri_memcpy(polyeri_ctx *ctx, void *dst, const void *src, size_t bytes, int to_device);
+/* Work buffers of the MP2, CC, gradient and k-point calls are kept for the
+ * next call, at most a quarter of the device's memory, until the device's
+ * last context is destroyed or an allocation of the library needs them.  This
+ * gives those not in use back to the device at once (of every context on it),
+ * for other allocators in the process or other processes; *bytes (optional) =
+ * how much. */
+int polyeri_release_work(polyeri_ctx *ctx, size_t *bytes);
 /* Device-to-device copy with the library's own streaming kernel (bytes a
  * multiple of 16); blocking.  A known-size reference for hardware counters. */
 int polyeri_device_copy(polyeri_ctx *ctx, void *dst, const void *src, size_t bytes);

@@ -427,6 +427,14 @@ class Context:
     def device_free(self, ptr):
         check(lib().polyeri_device_free(self.h, ptr))
 
+    def release_work(self):
+        """Give the work buffers that MP2, CC, gradient and k-point calls left
+        for the next call (at most a quarter of the device's memory) back to
+        the device, for torch or another process; returns their bytes."""
+        n = ctypes.c_size_t()
+        check(lib().polyeri_release_work(self.h, ctypes.byref(n)))
+        return n.value
+
     def to_device(self, dptr, arr):
         a = np.asfortranarray(arr, dtype=np.float64)
         check(lib().polyeri_memcpy(self.h, dptr, _p(a), a.nbytes, 1))

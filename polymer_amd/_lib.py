@@ -27,7 +27,7 @@ EXPORTS = [
     "polyeri_rys_nodes",
     "polyeri_rys_block", "polyeri_eri_gradient", "polyeri_eri_gradient_host", "polyeri_one_electron_gradient",
     "polyeri_one_electron_gradient_host", "polyeri_mp2_energy_periodic_mod", "polyeri_mp2_energy_periodic_qp",
-    "polyeri_mo_integrals", "polyeri_ccsd", "polyeri_cc",
+    "polyeri_mo_integrals", "polyeri_ccsd", "polyeri_cc", "polyeri_release_work",
 ]
 
 
@@ -152,6 +152,7 @@ def lib():
     L.polyeri_device_alloc.argtypes = [p, ctypes.c_size_t, ctypes.POINTER(p)]
     L.polyeri_device_free.argtypes = [p, p]
     L.polyeri_memcpy.argtypes = [p, p, p, ctypes.c_size_t, i]
+    L.polyeri_release_work.argtypes = [p, ctypes.POINTER(ctypes.c_size_t)]
     L.polyeri_fock_build_device.argtypes = [p, p, d, p, p, p]
     L.polyeri_device_copy.argtypes = [p, p, p, ctypes.c_size_t]
     L.polyeri_mlp_create.argtypes = [i, p, ctypes.c_ulonglong, ctypes.POINTER(p)]

@@ -2095,6 +2095,14 @@ int polyeri_device_free(polyeri_ctx* ctx, void* ptr) {
     return 0;
 }
 
+int polyeri_release_work(polyeri_ctx* ctx, size_t* bytes) {
+    if (!ctx) return fail(POLYERI_E_ARG, "polyeri_release_work: null context");
+    HIPCHK(hipSetDevice(ctx->device));
+    const size_t n = work_pool().release(ctx->device);
+    if (bytes) *bytes = n;
+    return 0;
+}
+
 int polyeri_memcpy(polyeri_ctx* ctx, void* dst, const void* src, size_t bytes, int to_device) {
     if (!ctx || !dst || !src) return fail(POLYERI_E_ARG, "polyeri_memcpy: null argument");
     HIPCHK(hipSetDevice(ctx->device));

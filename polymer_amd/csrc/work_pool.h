@@ -14,9 +14,12 @@ namespace polyeri {
 // handed out only while it is in use by nobody (mutex; the caller waits for
 // its streams before it gives a block back), and only for a request of nearly
 // its size, so that a call never holds noticeably more than it asked for.  At
-// most a quarter of a device's memory is kept idle; all of a device's idle
-// blocks go back when its last context ends and when an allocation of the
-// library fails (get, alloc; release for those that rocBLAS and rocSOLVER make).
+// most a quarter of a device's memory is kept idle ((H2O)12 cc-pVDZ MP2 works
+// in 46 GB), the oldest blocks making room for new ones; all of a device's
+// idle blocks go back when its last context ends, when an allocation of the
+// library fails (get, alloc; release for those that rocBLAS and rocSOLVER
+// make) and when the caller asks for it (polyeri_release_work), who alone
+// knows what others in the process or on the device need.
 //
 // Mem: the device's allocator, with static functions
 //   int device()                     the current device, negative on error
@@ -31,7 +34,7 @@ class WorkPool {
         int device;
     };
     std::mutex mu;
-    std::vector<Block> idle, used;
+    std::vector<Block> idle, used;        // idle: oldest first
     std::vector<int> contexts;            // live contexts per device
 
     // How much larger than a request its block may be: up to 64 KB more than
@@ -90,10 +93,19 @@ class WorkPool {
             if (used[i].p != p) continue;
             const Block b = used[i];
             used.erase(used.begin() + i);
-            if (idle_sum(b.device) + b.bytes <= Mem::total(b.device) / 4)
-                idle.push_back(b);
-            else
+            const size_t limit = Mem::total(b.device) / 4;
+            if (b.bytes > limit) {
                 Mem::free(b.p);
+                return;
+            }
+            size_t sum = idle_sum(b.device);
+            for (size_t k = 0; k < idle.size() && sum + b.bytes > limit;) {
+                if (idle[k].device != b.device) { ++k; continue; }
+                sum -= idle[k].bytes;
+                Mem::free(idle[k].p);
+                idle.erase(idle.begin() + k);
+            }
+            idle.push_back(b);
             return;
         }
     }

@@ -57,3 +57,19 @@ def test_reused_blocks_give_the_same_results():
         ctx.close()
     gc.collect()
     assert _free_bytes() > held
+
+
+def test_idle_blocks_are_given_back_on_request():
+    gc.collect()
+    print("case: idle work buffers released", flush=True)
+    ctx, e = _run(geometry.water_cluster(4, 1), "cc-pVDZ")
+    kept = _free_bytes()
+    n = ctx.release_work()
+    assert n > 400 << 20                       # the MO integrals alone are 0.8 GB
+    assert _free_bytes() - kept > n // 2
+    assert ctx.release_work() == 0
+    r = ctx.self_consistent_field(scfconv=1e-9, diis=2, scfcycles=100)
+    again = np.array(ctx.mp2_energy(r["co"], r["eps"], 0, r["iocc"], r["n_indep"]))
+    # the SCF's atomics change the last digits of the orbitals, and the energies to first order in them
+    assert np.max(np.abs(again - e[:2])) < 1e-8
+    ctx.close()

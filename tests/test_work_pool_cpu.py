@@ -137,14 +137,14 @@ def test_failed_allocation_reclaims_idle_blocks(shim):
     """Of the pool's own requests and of others', and only of that device."""
     for request in (shim.get, shim.raw):
         shim.start(100 * MB, 100 * MB)
-        shim.put(shim.get(20 * MB))
-        assert shim.idle(0) == 20 * MB
+        shim.put(shim.get(10 * MB))
+        assert shim.idle(0) == 10 * MB
         shim.set_device(1)
-        shim.put(shim.get(20 * MB))
+        shim.put(shim.get(10 * MB))
         shim.set_device(0)
-        assert request(90 * MB)
-        assert shim.idle(0) == 0 and shim.idle(1) == 20 * MB
-        assert not request(11 * MB)                         # really full
+        assert request(95 * MB)
+        assert shim.idle(0) == 0 and shim.idle(1) == 10 * MB
+        assert not request(6 * MB)                          # really full
 
 
 def test_release_gives_back_one_devices_idle_blocks(shim):
@@ -155,6 +155,21 @@ def test_release_gives_back_one_devices_idle_blocks(shim):
     assert shim.in_use(0) == 6 * MB                         # the block in use stays
     shim.put(q)
     assert shim.idle(0) == 6 * MB
+
+
+def test_idle_memory_is_bounded_and_the_newest(shim):
+    """Blocks of ever new sizes: what is kept never passes a quarter of the
+    device, and it is the blocks given back last."""
+    shim.start(400 * MB, 10 * MB)
+    shim.set_device(1)
+    shim.put(shim.get(MB))                                  # the other device's block is not the one to go
+    shim.set_device(0)
+    for k in range(12):
+        shim.put(shim.get((20 + 2 * k) * MB))
+        assert shim.idle(0) <= 100 * MB and shim.idle(0) == shim.in_use(0)
+    assert shim.idle(0) == (42 + 40) * MB and shim.idle(1) == MB
+    shim.put(shim.get(101 * MB))                            # too large to keep, and no reason to drop the others
+    assert shim.idle(0) == (42 + 40) * MB == shim.in_use(0)
 
 
 def test_every_allocation_of_the_library_reclaims():
