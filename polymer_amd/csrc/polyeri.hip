@@ -620,8 +620,10 @@ hipError_t polyeri_device_malloc(void** p, size_t bytes) { return (hipError_t)wo
 int polyeri_work_get(void** p, size_t bytes) { return work_pool().get(p, bytes); }
 void polyeri_work_put(void* p) { work_pool().put(p); }
 
-// Gives the current device's idle work buffers back; false where there are none.
+// Gives the current device's idle work buffers back; false where there are
+// none.  The failed allocation of a library is not the next launch's error.
 static bool release_idle_work() {
+    (void)hipGetLastError();
     const int device = HipMemory::device();
     return device >= 0 && work_pool().release(device) > 0;
 }
@@ -2337,9 +2339,11 @@ struct DevBuf {
     hipStream_t stream;
     explicit DevBuf(hipStream_t s) : stream(s) {}
     DevBuf(const DevBuf&) = delete;
-    ~DevBuf() {
+    ~DevBuf() { clear(); }
+    void clear() {
         if (!ptrs.empty()) (void)hipStreamSynchronize(stream);   // also where the call ended early
         for (void* p : ptrs) work_pool().put(p);
+        ptrs.clear();
     }
     template <typename T>
     int get(T** p, size_t n) {
@@ -3903,24 +3907,35 @@ static int mp2_periodic(polyeri_ctx* ctx, int kvc, const double* co, const doubl
     // all of them; at most half of what is left of the free memory, and an
     // eighth of the device's, for their TN
     const size_t more = std::min((freeb - freeb / 16 - need) / 2, totalb / 8) / (16 * (nTN + nB1));
-    const int kgrp = (int)std::min<size_t>(nk, 1 + more);
+    int kgrp = (int)std::min<size_t>(nk, 1 + more);
     int kfirst = 0;
     DevBuf buf(ctx->stream);
     double *dT, *dTNr, *dTNi, *dTOKr, *dTOKi, *dTVr, *dTVi, *dTOVr, *dTOVi, *dB1r, *dB1i, *dB2r, *dB2i, *dB3r, *dB3i,
         *dB4r, *dB4i, *dCr, *dCi, *dEps, *dAcc, *dQ = nullptr;
     double2* dCO;
     int* dPlim;
-    int rc;
-    if ((rc = buf.get(&dT, nT)) || (rc = buf.get(&dTNr, kgrp * nTN)) || (rc = buf.get(&dTNi, kgrp * nTN)) ||
-        (rc = buf.get(&dTOKr, nTOK)) || (rc = buf.get(&dTOKi, nTOK)) || (rc = buf.get(&dTVr, nTV)) ||
-        (rc = buf.get(&dTVi, nTV)) || (rc = buf.get(&dTOVr, nTOV)) || (rc = buf.get(&dTOVi, nTOV)) ||
-        (rc = buf.get(&dB1r, kgrp * nB1)) || (rc = buf.get(&dB1i, kgrp * nB1)) || (rc = buf.get(&dB2r, nB2)) ||
-        (rc = buf.get(&dB2i, nB2)) || (rc = buf.get(&dB3r, nB3)) || (rc = buf.get(&dB3i, nB3)) ||
-        (rc = buf.get(&dB4r, nB4)) || (rc = buf.get(&dB4i, nB4)) || (rc = buf.get(&dCr, nC)) ||
-        (rc = buf.get(&dCi, nC)) || (rc = buf.get(&dEps, (size_t)nc * nk)) || (rc = buf.get(&dAcc, 2)) ||
-        (rc = buf.get(&dCO, (size_t)nc * nc * nk)) || (rc = buf.get(&dPlim, (size_t)nk)) ||
-        (ng > 0 && (rc = buf.get(&dQ, (size_t)nk * ng))))
-        return rc;
+    auto take = [&](size_t g) {
+        int rc;
+        if ((rc = buf.get(&dT, nT)) || (rc = buf.get(&dTNr, g * nTN)) || (rc = buf.get(&dTNi, g * nTN)) ||
+            (rc = buf.get(&dTOKr, nTOK)) || (rc = buf.get(&dTOKi, nTOK)) || (rc = buf.get(&dTVr, nTV)) ||
+            (rc = buf.get(&dTVi, nTV)) || (rc = buf.get(&dTOVr, nTOV)) || (rc = buf.get(&dTOVi, nTOV)) ||
+            (rc = buf.get(&dB1r, g * nB1)) || (rc = buf.get(&dB1i, g * nB1)) || (rc = buf.get(&dB2r, nB2)) ||
+            (rc = buf.get(&dB2i, nB2)) || (rc = buf.get(&dB3r, nB3)) || (rc = buf.get(&dB3i, nB3)) ||
+            (rc = buf.get(&dB4r, nB4)) || (rc = buf.get(&dB4i, nB4)) || (rc = buf.get(&dCr, nC)) ||
+            (rc = buf.get(&dCi, nC)) || (rc = buf.get(&dEps, (size_t)nc * nk)) || (rc = buf.get(&dAcc, 2)) ||
+            (rc = buf.get(&dCO, (size_t)nc * nc * nk)) || (rc = buf.get(&dPlim, (size_t)nk)) ||
+            (ng > 0 && (rc = buf.get(&dQ, (size_t)nk * ng))))
+            return rc;
+        return 0;
+    };
+    int rc = take(kgrp);
+    if (rc == POLYERI_E_NOMEM) {      // not as much is to be had: exact blocks, one k-point at a time
+        buf.clear();
+        work_pool().release(ctx->device);
+        kgrp = 1;
+        rc = take(1);
+    }
+    if (rc) return rc;
     if (ng > 0) hipLaunchKernelGGL(k_fill, dim3(nblk((size_t)nk * ng)), dim3(256), 0, s, dQ, (size_t)nk * ng, 0.0);
     HIPCHK(hipMemcpyAsync(dCO, co, sizeof(double2) * (size_t)nc * nc * nk, hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(dEps, eps, 8 * (size_t)nc * nk, hipMemcpyHostToDevice, s));
