@@ -179,6 +179,8 @@ static int ensure_batch(polyeri_mlp* m, int batch) {
     for (float* p : m->d_z) (void)hipFree(p);
     for (float* p : m->d_a) (void)hipFree(p);
     (void)hipFree(m->d_part);
+    m->cap = 0;                       // no buffers until all of the new ones are there
+    m->d_part = nullptr;
     m->d_z.assign(m->nl + 1, nullptr);
     m->d_a.assign(m->nl + 1, nullptr);
     for (int l = 1; l <= m->nl; ++l) {

@@ -6,8 +6,12 @@ import os
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 
+import polymer_amd as pa
+from polymer_amd import geometry, guess
+from polymer_amd._lib import check, lib
 from tests.conftest import ROOT
 
 pytestmark = pytest.mark.gpu
@@ -140,3 +144,18 @@ def test_calls_at_the_end_of_memory(tmp_path, part):
     print(f"case: allocations refused, {part}", flush=True)
     r = subprocess.run([sys.executable, "-c", CHILD, so, part], cwd=ROOT, capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "bounded calls done" in r.stdout, r.stdout + r.stderr
+
+
+def test_network_after_a_batch_that_did_not_fit():
+    """A batch whose activations no device holds is refused before anything is
+    launched, and leaves a network that allocates again for the next one."""
+    print("case: network batch beyond the device's memory", flush=True)
+    ctx = pa.Context(pa.read_basis("STO-3G", geometry.water()))
+    net = guess.MLP([8, 4096, 4096, 5], seed=3)
+    x = np.random.default_rng(1).standard_normal((40, 8)).astype(np.float32)
+    y = guess.mlp_forward(net, ctx, x)
+    d = ctx.device_alloc(1 << 20)
+    with pytest.raises(pa.PolyeriError):
+        check(lib().polyeri_mlp_forward(net.h, d, 2 ** 30, d))
+    ctx.device_free(d)
+    assert np.array_equal(guess.mlp_forward(net, ctx, x), y)
