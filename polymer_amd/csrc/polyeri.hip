@@ -284,7 +284,7 @@ enum { LAUNCH_AUTO = 0, LAUNCH_REG = 1, LAUNCH_COOP = 2, LAUNCH_SEG = 3, LAUNCH_
 static const int RYS_NMAX_EXPORT = 5;
 // Items per bra-row segment of the segment kernel (at most), and the number
 // of segments a list's primitive quartets are spread over (at least); the
-// Rys classes' segments and least items (make_segments).
+// Rys classes' segments and least items (SegmentLists).
 static const int kSegItems = 2048, kSegMin = 256;
 static const double kSegTarget = 4096.0;
 static const long long kSegTargetRys = 1024, kSegMinRys = 16;
@@ -310,110 +310,134 @@ static int segment_split(double bp, double kp, double list_total, double ctx_tot
     return ls;
 }
 
-// Bra-row segments of a work list for the segment kernels: each segment is
-// part of one row, at most kSegItems items and about `target` primitive
-// quartets (the row's bra primitive count times each ket's), with target =
-// the list's primitive quartets / kSegTarget, but at least one pass of a
-// block (kSegMin lanes: shorter segments pay more for their row flush than
-// they gain in balance) where the row has them; ordered by
-// primitive quartets, largest first, so that the blocks launched last are
-// the short ones.  The items of a segment are shared by equally many lanes
-// (segment_split; split = the primitive quartets of all lists, 0: one lane
-// each), so a row is also cut where that changes.  pairs / bra / kets /
-// bstart: the list's pair data, bra ids by row, ket ids and bucket starts of
-// the ket class.  balanced = false: rows cut every kSegItems lanes, in row
-// order (the autotuner keeps whichever form is faster per list).  rys: the
+// Bra-row segments of a work list for the segment kernels, in two forms (the
+// autotuner keeps whichever is faster per list), with the largest ket bound of
+// each segment: a density-screened build skips a segment whole whose bra bound
+// x this x the largest |D| block is below the threshold.
+// Balanced: each segment is part of one row, at most kSegItems items and about
+// `target` primitive quartets (the row's bra primitive count times each
+// ket's), with target = the list's primitive quartets / kSegTarget, but at
+// least one pass of a block (kSegMin lanes: shorter segments pay more for
+// their row flush than they gain in balance) where the row has them; ordered
+// by primitive quartets, largest first, so that the blocks launched last are
+// the short ones.  Unbalanced: rows cut every kSegItems lanes, in row order.
+// The items of a segment are shared by equally many lanes (segment_split;
+// split = the primitive quartets of all lists, 0: one lane each), so a row is
+// also cut where that changes.  pairs / bra / kets / bstart: the list's pair
+// data, bra ids by row, ket ids and bucket starts of the ket class.  rys: the
 // list of a Rys class, whose items take 3 or 6 lanes of each of 1 to 8
 // variants (so up to 2^4 groups of lanes may share one) and far outweigh a
 // row flush: short lists are cut finer, into about kSegTargetRys segments of
 // at least kSegMinRys items, four blocks a CU ((H2O)16 cc-pVDZ, 103 -> 1092
 // segments of (dd|dp): 0.31 -> 0.15 ms; lists of 1000 segments and more lose
 // to the flushes, (dp|pp) of 2066 -> 3599: 0.67 -> 0.74 ms, and stay).
-static std::vector<SegDesc> make_segments(const WorkList& l, const std::vector<PairInfo>& pairs,
-                                          const std::vector<int>& bra, const std::vector<int>& kets,
-                                          const std::vector<int>& bstart, double split, bool balanced = true,
-                                          bool rys = false) {
-    const int nb = l.nbucket;
-    std::vector<double> knp(nb, 0.0);
-    for (int b = 0; b + 1 < (int)bstart.size() && b < nb; ++b) knp[b] = pairs[kets[bstart[b]]].nprim;
-    const double target = balanced ? l.prim_quartets / kSegTarget : 1e300;
-    const int least = rys ? (int)std::clamp<long long>(l.nwork / kSegTargetRys, kSegMinRys, kSegMin) : kSegMin;
-    std::vector<std::pair<double, SegDesc>> segs;
-    for (int r = 0; r < l.nrows; ++r) {
-        const double bp = pairs[bra[r]].nprim;
-        const int* rb = l.rb.data() + (size_t)r * (nb + 1);
-        long long t = l.row[r];
-        int n = 0, ls = 0;
-        double cost = 0.0;
-        auto flush = [&] {
-            if (n > 0) segs.push_back({cost, SegDesc{t, r, n, ls}});
-            t += n; n = 0; cost = 0.0;
-        };
-        for (int b = 0; b < nb; ++b) {
-            int cnt = rb[b + 1] - rb[b];
-            if (cnt <= 0) continue;
-            const double ci = bp * knp[b];
-            const int lb = split > 0.0 ? segment_split(bp, knp[b], l.prim_quartets, split, rys ? 4 : 6) : 0;
-            if (lb != ls) flush();
-            ls = lb;
-            const int nmax = kSegItems >> ls, nmin = std::max(1, least >> ls);
-            while (cnt > 0) {
-                int take = std::min(cnt, nmax - n);
-                if (ci > 0.0)
-                    take = (int)std::min<double>(take, std::max<double>(nmin - n, std::ceil((target - cost) / ci)));
-                take = std::max(take, 1);
-                n += take; cost += take * ci; cnt -= take;
-                if (n >= nmax || (n >= nmin && cost >= target)) flush();
+// The lists are a large part of a context's creation, so one walk over a row
+// builds both forms and their bounds, the lanes are looked up by the row's
+// primitive count, and the vectors are kept from list to list (a context of
+// (H2O)16 cc-pVDZ 74 -> 60 ms, of (H2O)5 6-31G** 5.6 -> 4.1 ms, a millisecond
+// of each from the Boys table made once).
+struct SegmentLists {
+    std::vector<SegDesc> out;          // nseg balanced, nsegc unbalanced, then a bound (double) each
+    int nseg = 0, nsegc = 0;
+    bool share[2] = {false, false};    // whether some of the nseg (nsegc) share items between lanes
+
+    // kq: the kets' Schwarz bounds in ket order.  They descend inside a
+    // bucket, so the largest of a range is its first.
+    void build(const WorkList& l, const std::vector<PairInfo>& pairs, const std::vector<int>& bra,
+               const std::vector<int>& kets, const std::vector<int>& bstart, const std::vector<double>& kq,
+               double split, bool rys = false) {
+        const int nb = l.nbucket;
+        knp.assign(nb, 0.0);
+        for (int b = 0; b + 1 < (int)bstart.size() && b < nb; ++b) knp[b] = pairs[kets[bstart[b]]].nprim;
+        const double target = l.prim_quartets / kSegTarget;
+        const int least = rys ? (int)std::clamp<long long>(l.nwork / kSegTargetRys, kSegMinRys, kSegMin) : kSegMin;
+        segs.clear(); bound.clear(); order.clear(); segc.clear(); boundc.clear(); lanes.clear();
+        share[0] = share[1] = false;
+        const int* lb = nullptr;       // lanes (log2) of each bucket's items: the row's primitive count decides
+        int np_last = -1;
+        for (int r = 0; r < l.nrows; ++r) {
+            if (l.row[r] == l.row[r + 1]) continue;
+            const int np = pairs[bra[r]].nprim;
+            if (np != np_last) {
+                std::vector<int>& v = lanes[np];
+                if (v.empty()) {
+                    v.assign(nb, 0);
+                    for (int b = 0; b < nb && split > 0.0; ++b)
+                        v[b] = segment_split(np, knp[b], l.prim_quartets, split, rys ? 4 : 6);
+                }
+                lb = v.data();
+                np_last = np;
+            }
+            const int* rb = l.rb.data() + (size_t)r * (nb + 1);
+            const int* rf = l.rf.empty() ? nullptr : l.rf.data() + (size_t)r * nb;
+            const auto first_bound = [&](int b, int item) { return kq[bstart[b] + (rf ? rf[b] : 0) + item - rb[b]]; };
+            int t = 0, n = 0, ls = 0;
+            double cost = 0.0, q = 0.0;
+            const auto flush = [&] {
+                if (n > 0) {
+                    order.push_back({cost, (int)segs.size()});
+                    segs.push_back(SegDesc{l.row[r] + t, r, n, ls});
+                    bound.push_back(q);
+                    share[0] |= ls > 0;
+                }
+                t += n; n = 0; cost = q = 0.0;
+            };
+            for (int b = 0; b < nb; ++b) {
+                int cnt = rb[b + 1] - rb[b];
+                if (cnt <= 0) continue;
+                const double ci = np * knp[b];
+                if (lb[b] != ls) flush();
+                ls = lb[b];
+                const int nmax = kSegItems >> ls, nmin = std::max(1, least >> ls);
+                while (cnt > 0) {
+                    int take = std::min(cnt, nmax - n);
+                    if (take > nmin - n && ci > 0.0)
+                        take = (int)std::min<double>(take, std::max<double>(nmin - n, std::ceil((target - cost) / ci)));
+                    take = std::max(take, 1);
+                    q = std::max(q, first_bound(b, t + n));
+                    n += take; cost += take * ci; cnt -= take;
+                    if (n >= nmax || (n >= nmin && cost >= target)) flush();
+                }
+            }
+            flush();
+            for (int b = 0, e; b < nb; b = e) {           // buckets b .. e - 1: equally many lanes
+                for (e = b + 1; e < nb && lb[e] == lb[b]; ++e) {}
+                int x = b;
+                for (int m = rb[b], end; m < rb[e]; m = end) {
+                    end = std::min(m + (kSegItems >> lb[b]), rb[e]);
+                    double qc = 0.0;
+                    while (true) {
+                        if (rb[x] < rb[x + 1]) qc = std::max(qc, first_bound(x, std::max(m, rb[x])));
+                        if (rb[x + 1] >= end) break;
+                        ++x;
+                    }
+                    segc.push_back(SegDesc{l.row[r] + m, r, end - m, lb[b]});
+                    boundc.push_back(qc);
+                    share[1] |= lb[b] > 0;
+                    if (rb[x + 1] == end) ++x;
+                }
             }
         }
-        flush();
-    }
-    if (balanced)
-        std::stable_sort(segs.begin(), segs.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
-    std::vector<SegDesc> out(segs.size());
-    for (size_t i = 0; i < segs.size(); ++i) out[i] = segs[i].second;
-    return out;
-}
-static bool shares_items(const std::vector<SegDesc>& segs) {
-    return std::any_of(segs.begin(), segs.end(), [](const SegDesc& s) { return s.ls > 0; });
-}
-
-// Largest ket Schwarz bound kq over the items of each segment.  A row's
-// items cover one contiguous range of ket positions per bucket (the
-// decode_in_row mapping), so a sparse table of range maxima over the ket
-// order answers each range.  With a density-screened build a segment whose
-// bra bound x this x the largest |D| block is below the threshold holds no
-// surviving item and is skipped whole.
-static std::vector<double> segment_ket_bounds(const WorkList& l, const std::vector<SegDesc>& segs,
-                                              const std::vector<int>& kets, const std::vector<int>& bstart,
-                                              const std::vector<double>& kq) {
-    const int P = (int)kets.size();
-    std::vector<double> out(segs.size(), 0.0);
-    if (P == 0) return out;
-    std::vector<std::vector<double>> sp(1, std::vector<double>(P));
-    for (int i = 0; i < P; ++i) sp[0][i] = kq[kets[i]];
-    for (int k = 1; (1 << k) <= P; ++k) {
-        sp.emplace_back(P - (1 << k) + 1);
-        for (int i = 0; i + (1 << k) <= P; ++i) sp[k][i] = std::max(sp[k - 1][i], sp[k - 1][i + (1 << (k - 1))]);
-    }
-    const int nb = l.nbucket;
-    for (size_t s = 0; s < segs.size(); ++s) {
-        const SegDesc& sg = segs[s];
-        const int* rb = l.rb.data() + (size_t)sg.row * (nb + 1);
-        const long long l0 = sg.t0 - l.row[sg.row], l1 = l0 + sg.n;
-        double m = 0.0;
-        for (int b = 0; b < nb && b + 1 < (int)bstart.size(); ++b) {
-            const long long lo = std::max<long long>(l0, rb[b]), hi = std::min<long long>(l1, rb[b + 1]);
-            if (lo >= hi) continue;
-            const int first = l.rf.empty() ? 0 : l.rf[(size_t)sg.row * nb + b];
-            const int p0 = bstart[b] + first + (int)(lo - rb[b]), p1 = p0 + (int)(hi - lo);
-            const int k = 31 - __builtin_clz((unsigned)(p1 - p0));
-            m = std::max(m, std::max(sp[k][p0], sp[k][p1 - (1 << k)]));
+        std::stable_sort(order.begin(), order.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
+        nseg = (int)segs.size();
+        nsegc = (int)segc.size();
+        const size_t ns = segs.size() + segc.size();
+        out.resize(ns + (ns + 1) / 2);
+        double* q = reinterpret_cast<double*>(out.data() + ns);
+        for (size_t i = 0; i < segs.size(); ++i) {
+            out[i] = segs[order[i].second];
+            q[i] = bound[order[i].second];
         }
-        out[s] = m;
+        std::copy(segc.begin(), segc.end(), out.begin() + nseg);
+        std::copy(boundc.begin(), boundc.end(), q + nseg);
     }
-    return out;
-}
+
+  private:
+    std::vector<double> knp, bound, boundc;
+    std::vector<SegDesc> segs, segc;
+    std::vector<std::pair<double, int>> order;            // cost, place in segs
+    std::unordered_map<int, std::vector<int>> lanes;
+};
 
 struct LaunchCfg {
     int kind = LAUNCH_AUTO, block = 256, grid = 0;
@@ -433,8 +457,8 @@ struct ClassPairWork {
     int* d_rf;             // FP32 list: nrows x nbucket first kets (else null)
     int2* d_items;         // density-screened items (capacity nwork), allocated on first use
     SegDesc* d_seg;        // bra-row segments (molecular lists): nseg cost-balanced ones, then
-    int nseg, nsegc;       // nsegc of kSegItems items each (make_segments)
-    double* d_segq;        // per segment of d_seg: the largest ket bound (segment_ket_bounds)
+    int nseg, nsegc;       // nsegc of kSegItems lanes each (SegmentLists)
+    double* d_segq;        // per segment of d_seg: the largest ket bound (in d_seg's allocation)
     bool share[2];         // whether some of the nseg (nsegc) segments share items between lanes
     LaunchCfg cfg;         // launch shape (autotuned or default)
     int prec;              // 0: FP64, 1: FP32 (mixed precision)
@@ -634,6 +658,24 @@ static int dalloc(T** p, size_t n) {
     const hipError_t e = polyeri_device_malloc((void**)p, n * sizeof(T));
     if (e != hipSuccess) return fail(POLYERI_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     return 0;
+}
+
+// A list's segments and their ket bounds on the device, in one allocation.
+static int upload_segments(const SegmentLists& sl, SegDesc** d_seg, double** d_segq, int* nseg, int* nsegc) {
+    if ((long long)sl.nseg + sl.nsegc > 0x7fffffffLL) return fail(POLYERI_E_ARG, "too many segments");
+    const int rc = dalloc(d_seg, sl.out.size());
+    if (rc) return rc;
+    HIPCHK(hipMemcpy(*d_seg, sl.out.data(), sl.out.size() * sizeof(SegDesc), hipMemcpyHostToDevice));
+    *nseg = sl.nseg;
+    *nsegc = sl.nsegc;
+    *d_segq = reinterpret_cast<double*>(*d_seg + sl.nseg + sl.nsegc);
+    return 0;
+}
+// The bounds q of pairs ids, in their order.
+static std::vector<double> bounds_of(const std::vector<int>& ids, const std::vector<double>& q) {
+    std::vector<double> out(ids.size());
+    for (size_t i = 0; i < ids.size(); ++i) out[i] = q[ids[i]];
+    return out;
 }
 
 static int ensure_onee_device(polyeri_ctx* c) {
@@ -938,7 +980,6 @@ static void free_ctx(polyeri_ctx* c) {
         if (w.d_rf) (void)hipFree(w.d_rf);
         if (w.d_items) (void)hipFree(w.d_items);
         if (w.d_seg) (void)hipFree(w.d_seg);
-        (void)hipFree(w.d_segq); (void)hipFree(w.gc.d_segq);
         if (w.gc.d_row) (void)hipFree(w.gc.d_row);
         if (w.gc.d_rb) (void)hipFree(w.gc.d_rb);
         if (w.gc.d_seg) (void)hipFree(w.gc.d_seg);
@@ -1061,6 +1102,9 @@ static int build_gc_lists(polyeri_ctx* c) {
     if ((rc = dalloc(&c->d_gksoa, soa.size()))) return rc;
     HIPCHK(hipMemcpy(c->d_gksoa, soa.data(), soa.size() * sizeof(double), hipMemcpyHostToDevice));
     c->gkfs = (long long)P;
+    SegmentLists sl;
+    std::vector<double> kq[2];
+    for (int Y : {0, 1}) kq[Y] = bounds_of(kets[Y], gQ);
     for (const WorkList& l : wl) {
         if (l.nwork <= 0) continue;
         const int la = kPairL[l.X][0], lc = kPairL[l.Y][0];
@@ -1071,27 +1115,16 @@ static int build_gc_lists(polyeri_ctx* c) {
         for (ClassPairWork& x : c->work)
             if (x.X == l.X && x.Y == l.Y && x.prec == 0) w = &x;
         if (!w) continue;
-        std::vector<SegDesc> segs = make_segments(l, gp, cls[l.X], kets[l.Y], bst[l.Y], c->prim_quartets);
-        const std::vector<SegDesc> segc = make_segments(l, gp, cls[l.X], kets[l.Y], bst[l.Y], c->prim_quartets, false);
-        if (segs.size() + segc.size() > 0x7fffffffu) return fail(POLYERI_E_ARG, "too many segments");
         auto& g = w->gc;
+        sl.build(l, gp, cls[l.X], kets[l.Y], bst[l.Y], kq[l.Y], c->prim_quartets);
+        if ((rc = upload_segments(sl, &g.d_seg, &g.d_segq, &g.nseg, &g.nsegc))) return rc;
         g.nwork = l.nwork; g.nrows = l.nrows; g.nbucket = l.nbucket;
-        g.nseg = (int)segs.size(); g.nsegc = (int)segc.size();
-        segs.insert(segs.end(), segc.begin(), segc.end());
-        {
-            const std::vector<double> sq = segment_ket_bounds(l, segs, kets[l.Y], bst[l.Y], gQ);
-            if ((rc = dalloc(&g.d_segq, sq.size()))) return rc;
-            HIPCHK(hipMemcpy(g.d_segq, sq.data(), sq.size() * sizeof(double), hipMemcpyHostToDevice));
-        }
         g.d_bra = c->d_gbra[l.X]; g.d_ket = c->d_gket[l.Y]; g.d_bstart = c->d_gbstart[l.Y];
         g.d_bsoa = c->d_gbsoa[l.Y];
         g.prim_quartets = l.prim_quartets;
-        if ((rc = dalloc(&g.d_row, l.row.size())) || (rc = dalloc(&g.d_rb, l.rb.size())) ||
-            (rc = dalloc(&g.d_seg, segs.size())))
-            return rc;
+        if ((rc = dalloc(&g.d_row, l.row.size())) || (rc = dalloc(&g.d_rb, l.rb.size()))) return rc;
         HIPCHK(hipMemcpy(g.d_row, l.row.data(), l.row.size() * sizeof(long long), hipMemcpyHostToDevice));
         if (!l.rb.empty()) HIPCHK(hipMemcpy(g.d_rb, l.rb.data(), l.rb.size() * sizeof(int), hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(g.d_seg, segs.data(), segs.size() * sizeof(SegDesc), hipMemcpyHostToDevice));
         w->gc_on = 1;
     }
     // Shell-pair bras of the classes (pp) (ds) (dp) against group-pair kets
@@ -1124,42 +1157,64 @@ static int build_gc_lists(polyeri_ctx* c) {
         for (ClassPairWork& x : c->work)
             if (x.X == l.X && x.Y == l.Y && x.prec == 0) w = &x;
         if (!w || w->gc.nwork > 0) continue;
-        std::vector<SegDesc> segs = make_segments(l, cp, cid[l.X], ck[l.Y], cb[l.Y], c->prim_quartets);
-        const std::vector<SegDesc> segc = make_segments(l, cp, cid[l.X], ck[l.Y], cb[l.Y], c->prim_quartets, false);
-        if (segs.size() + segc.size() > 0x7fffffffu) return fail(POLYERI_E_ARG, "too many segments");
         auto& g = w->gc;
         g.kind = 1;
-        {
-            std::vector<SegDesc> all(segs);
-            all.insert(all.end(), segc.begin(), segc.end());
-            const std::vector<double> sq = segment_ket_bounds(l, all, ck[l.Y], cb[l.Y], cq);
-            if ((rc = dalloc(&g.d_segq, sq.size()))) return rc;
-            HIPCHK(hipMemcpy(g.d_segq, sq.data(), sq.size() * sizeof(double), hipMemcpyHostToDevice));
-        }
+        sl.build(l, cp, cid[l.X], ck[l.Y], cb[l.Y], kq[l.Y], c->prim_quartets);
+        if ((rc = upload_segments(sl, &g.d_seg, &g.d_segq, &g.nseg, &g.nsegc))) return rc;
         g.nwork = l.nwork; g.nrows = l.nrows; g.nbucket = l.nbucket;
-        g.nseg = (int)segs.size(); g.nsegc = (int)segc.size();
-        segs.insert(segs.end(), segc.begin(), segc.end());
         g.d_bra = c->d_class_ids[l.X]; g.d_ket = c->d_gket[l.Y]; g.d_bstart = c->d_gbstart[l.Y];
         g.d_bsoa = c->d_gbsoa[l.Y];
         g.prim_quartets = l.prim_quartets;
-        if ((rc = dalloc(&g.d_row, l.row.size())) || (rc = dalloc(&g.d_rb, l.rb.size())) ||
-            (rc = dalloc(&g.d_seg, segs.size())))
-            return rc;
+        if ((rc = dalloc(&g.d_row, l.row.size())) || (rc = dalloc(&g.d_rb, l.rb.size()))) return rc;
         HIPCHK(hipMemcpy(g.d_row, l.row.data(), l.row.size() * sizeof(long long), hipMemcpyHostToDevice));
         if (!l.rb.empty()) HIPCHK(hipMemcpy(g.d_rb, l.rb.data(), l.rb.size() * sizeof(int), hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(g.d_seg, segs.data(), segs.size() * sizeof(SegDesc), hipMemcpyHostToDevice));
         w->gc_on = 0;
     }
     return 0;
+}
+
+// The Boys values on their grid, BOYS_NT x BOYS_NM: constants, tabulated once
+// (1 ms; a context of five waters takes 5).
+static const std::vector<double>& boys_values() {
+    static const std::vector<double> table = [] {
+        std::vector<double> t;
+        boys_table(t);
+        return t;
+    }();
+    return table;
+}
+// The device's layouts of them: the table, then the aligned per-L rows of the
+// thread kernels, then the coarse per-L rows (eri_engine.h).
+static const std::vector<double>& boys_device_values() {
+    static_assert(BOYS_LC - 2 + 9 < BOYS_NM && BOYS_LA - 2 + 7 < BOYS_NM && 3 * (BOYS_CNT - 1) < BOYS_NT,
+                  "Boys rows out of the table");
+    static const std::vector<double> layouts = [] {
+        const std::vector<double>& boys = boys_values();
+        std::vector<double> dev(boys);
+        dev.resize((size_t)BOYS_COFF + (size_t)BOYS_LC * BOYS_CROWS, 0.0);
+        auto row = [&](double* out, int n, int L, int i) {
+            const double* f = boys.data() + (size_t)i * BOYS_NM + (L > 0 ? L - 1 : 0);
+            double fact = 1.0;
+            for (int k = 0; k < n; ++k) {
+                out[k] = f[k] / fact;
+                fact *= k + 1;
+            }
+        };
+        for (int L = 0; L < BOYS_LA; ++L)
+            for (int i = 0; i < BOYS_NT; ++i) row(dev.data() + BOYS_AOFF + ((size_t)L * BOYS_NT + i) * 8, 8, L, i);
+        for (int L = 0; L < BOYS_LC; ++L)
+            for (int j = 0; j < BOYS_CNT; ++j)
+                row(dev.data() + BOYS_COFF + (size_t)L * BOYS_CROWS + j * 10, 10, L, 3 * j);
+        return dev;
+    }();
+    return layouts;
 }
 
 static int build_ctx(polyeri_ctx* c) {
     std::string err;
     if (extract_shells(c->rb, c->ib, err)) return fail(POLYERI_E_BASIS, err);
     if (c->pbc) {
-        std::vector<double> boys0;
-        boys_table(boys0);
-        c->rc1 = reduced_cel1(c->ib, c->period, c->cel1, boys0);
+        c->rc1 = reduced_cel1(c->ib, c->period, c->cel1, boys_values());
         build_pairs_cells(c->ib, c->opts.prim_tol, c->period, c->rc1, c->pairs, c->prims, c->pcell);
     } else {
         build_pairs(c->ib, c->opts.prim_tol, c->pairs, c->prims);
@@ -1183,31 +1238,12 @@ static int build_ctx(polyeri_ctx* c) {
         meta[i] = {p.prim_off, p.nprim, c->ib.shells[p.a].f0, c->ib.shells[p.b].f0};
         ab[4 * i] = p.ABx; ab[4 * i + 1] = p.ABy; ab[4 * i + 2] = p.ABz; ab[4 * i + 3] = 0;
     }
-    std::vector<double> boys;
-    boys_table(boys);
+    const std::vector<double>& boys = boys_values();
     int rc;
     if ((rc = dalloc(&c->d_prims, c->prims.size()))) return rc;
     if ((rc = dalloc(&c->d_meta, np))) return rc;
     if ((rc = dalloc(&c->d_ab, 4 * (size_t)np))) return rc;
-    // device copy: the BOYS_NT x BOYS_NM table, then the aligned per-L rows
-    // of the thread kernels, then the coarse per-L rows (eri_engine.h)
-    static_assert(BOYS_LC - 2 + 9 < BOYS_NM && BOYS_LA - 2 + 7 < BOYS_NM && 3 * (BOYS_CNT - 1) < BOYS_NT,
-                  "Boys rows out of the table");
-    std::vector<double> boys_dev(boys);
-    boys_dev.resize((size_t)BOYS_COFF + (size_t)BOYS_LC * BOYS_CROWS, 0.0);
-    auto row = [&](double* out, int n, int L, int i) {
-        const double* f = boys.data() + (size_t)i * BOYS_NM + (L > 0 ? L - 1 : 0);
-        double fact = 1.0;
-        for (int k = 0; k < n; ++k) {
-            out[k] = f[k] / fact;
-            fact *= k + 1;
-        }
-    };
-    for (int L = 0; L < BOYS_LA; ++L)
-        for (int i = 0; i < BOYS_NT; ++i) row(boys_dev.data() + BOYS_AOFF + ((size_t)L * BOYS_NT + i) * 8, 8, L, i);
-    for (int L = 0; L < BOYS_LC; ++L)
-        for (int j = 0; j < BOYS_CNT; ++j)
-            row(boys_dev.data() + BOYS_COFF + (size_t)L * BOYS_CROWS + j * 10, 10, L, 3 * j);
+    const std::vector<double>& boys_dev = boys_device_values();
     if ((rc = dalloc(&c->d_boys, boys_dev.size()))) return rc;
     if ((rc = dalloc(&c->d_Q, np))) return rc;
     if ((rc = dalloc(&c->d_ref, nbf))) return rc;
@@ -1312,6 +1348,9 @@ static int build_ctx(polyeri_ctx* c) {
     c->quartets = 0; c->prim_quartets = 0; c->model_flops = 0;
     double all = 0.0;
     for (const WorkList& l : wl) all += l.prim_quartets;
+    SegmentLists sl;
+    std::vector<double> kq[NPAIRCLASS];
+    for (int Y = 0; Y < NPAIRCLASS; ++Y) kq[Y] = bounds_of(c->ket_ids[Y], c->Q);
     for (const WorkList& l : wl) {
         ClassPairWork w;
         w.X = l.X; w.Y = l.Y;
@@ -1346,21 +1385,9 @@ static int build_ctx(polyeri_ctx* c) {
         // split the light classes.
         if (!c->pbc && l.nwork > 0 && (!l.prec || polyeri_rys_class(w.la, w.lb, w.lc, w.ld))) {
             const bool rys = polyeri_rys_class(w.la, w.lb, w.lc, w.ld);
-            std::vector<SegDesc> segs =
-                make_segments(l, c->pairs, c->class_ids[l.X], c->ket_ids[l.Y], c->bstart[l.Y], all, true, rys);
-            const std::vector<SegDesc> segc =
-                make_segments(l, c->pairs, c->class_ids[l.X], c->ket_ids[l.Y], c->bstart[l.Y], all, false, rys);
-            if (segs.size() + segc.size() > 0x7fffffffu) return fail(POLYERI_E_ARG, "too many segments");
-            w.nseg = (int)segs.size();
-            w.nsegc = (int)segc.size();
-            w.share[0] = shares_items(segs);
-            w.share[1] = shares_items(segc);
-            segs.insert(segs.end(), segc.begin(), segc.end());
-            if ((rc = dalloc(&w.d_seg, segs.size()))) return rc;
-            HIPCHK(hipMemcpy(w.d_seg, segs.data(), segs.size() * sizeof(SegDesc), hipMemcpyHostToDevice));
-            const std::vector<double> sq = segment_ket_bounds(l, segs, c->ket_ids[l.Y], c->bstart[l.Y], c->Q);
-            if ((rc = dalloc(&w.d_segq, sq.size()))) return rc;
-            HIPCHK(hipMemcpy(w.d_segq, sq.data(), sq.size() * sizeof(double), hipMemcpyHostToDevice));
+            sl.build(l, c->pairs, c->class_ids[l.X], c->ket_ids[l.Y], c->bstart[l.Y], kq[l.Y], all, rys);
+            if ((rc = upload_segments(sl, &w.d_seg, &w.d_segq, &w.nseg, &w.nsegc))) return rc;
+            std::copy(sl.share, sl.share + 2, w.share);
         }
         if (l.prec) {
             if ((rc = dalloc(&w.d_rf, l.rf.size()))) return rc;
@@ -3317,8 +3344,7 @@ static void one_electron_cells(const polyeri_ctx* c, std::vector<double>& S, std
     const int nbf = ib.nbf, nc = c->rb.ncgs, ncell = 2 * c->cel1 + 1;
     const size_t c2 = (size_t)nc * nc;
     S.assign(c2 * ncell, 0.0); T.assign(c2 * ncell, 0.0); N.assign(c2 * ncell, 0.0);
-    std::vector<double> boys;
-    boys_table(boys);
+    const std::vector<double>& boys = boys_values();
     std::vector<int> z;
     std::vector<double> xyz;
     for (int k = -c->cel2; k <= c->cel2; ++k)
@@ -4501,8 +4527,7 @@ static int one_electron_gradient_ib(const IntBasis& ib, const RefBasis& rb, cons
             D[(size_t)mu * nbf + nu] = sc * p_c[r];
             W[(size_t)mu * nbf + nu] = sc * w_c[r];
         }
-    std::vector<double> boys;
-    boys_table(boys);
+    const std::vector<double>& boys = boys_values();
     one_electron_gradient(ib, at, boys, D.data(), W.data(), grad);
     for (int i = 0; i < 3 * rb.natom; ++i)
         if (!std::isfinite(grad[i])) return fail(POLYERI_E_NONFINITE, "one-electron gradient: non-finite value");
