@@ -1429,13 +1429,13 @@ int polyeri_gemm_launch(int mode, int M, int N, int K, const double* A, long sam
                         hipStream_t stream);
 // Planar complex products C_b = A_b B_b (A real when Ai is null), same
 // strides for the real and imaginary planes, k contiguous in A and n in B
-// (kgemm.hip).  nci > 0 splits the columns of B and C as (n / nci, n % nci)
+// (kgemm.hip; C linkage for its test).  nci > 0 splits the columns of B and C as (n / nci, n % nci)
 // with outer strides sbo / sco, mci > 0 the rows of C as (m / mci, m % mci)
 // with outer stride smo.
-int polyeri_zgemm_launch(int mode, int M, int N, int K, const double* Ar, const double* Ai, long sam, long sA,
-                         const double* Br, const double* Bi, long sbk, long sB, double* Cr, double* Ci, long scm,
-                         long scn, long sC, int batch, hipStream_t stream, int nci = 0, long sbo = 0, long sco = 0,
-                         int mci = 0, long smo = 0);
+extern "C" int polyeri_zgemm_launch(int mode, int M, int N, int K, const double* Ar, const double* Ai, long sam,
+                                    long sA, const double* Br, const double* Bi, long sbk, long sB, double* Cr,
+                                    double* Ci, long scm, long scn, long sC, int batch, hipStream_t stream,
+                                    int nci = 0, long sbo = 0, long sco = 0, int mci = 0, long smo = 0);
 // Density screening (kscreen.hip): shell-block maxima of |D|, and the
 // compaction of one work list to the items whose bound
 // Q_ab Q_cd max(|D| over the six blocks the quartet reads) reaches tol.

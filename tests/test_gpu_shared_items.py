@@ -105,9 +105,11 @@ D    2   1.00
 def test_shared_rys_items_match_oracle(tmp_path, atoms):
     """The Rys classes with 8 (six-lane members) and 16 (three-lane members)
     lane groups an item, against the oracle and with the screen that keeps
-    every quartet; and the mixed-precision lists.  Tolerance as above; FP32
-    lists: integrals below the cut 1 times 2^-24 per operation of a sum of at
-    most 10^3 terms an element, 1e-3 of the largest element."""
+    every quartet; and the mixed-precision lists, part and all of the quartets
+    in FP32.  Tolerance as above; FP32: an integral sums at most 144 primitive
+    quartets of 3 to 5 roots, about 512 terms rounded to 2^-24 with errors of
+    either sign, sqrt(512) 2^-24 of the sums that the density's magnitudes
+    give (1.4e-6 of them; 2e-8 measured)."""
     path = str(tmp_path / "deep")
     with open(path, "w") as f:
         f.write(DEEP_BASIS.format(el="Ne"))
@@ -126,7 +128,11 @@ def test_shared_rys_items_match_oracle(tmp_path, atoms):
     assert np.max(np.abs(j - jr)) < 1e-10 and np.max(np.abs(k - kr)) < 1e-10
     js, ks = ctx.fourindex_eri(p, dens_tol=1e-290)
     assert np.max(np.abs(js - jr)) < 1e-10 and np.max(np.abs(ks - kr)) < 1e-10
-    mixed = pa.Context(b, schwarz_tol=0.0, precision=pa.MIXED, mixed_cut=1.0)
-    jm, km = mixed.fourindex_eri(p)
-    assert np.max(np.abs(jm - jr)) < 1e-3 * np.max(np.abs(jr))
-    assert np.max(np.abs(km - kr)) < 1e-3 * np.max(np.abs(kr))
+    ja, ka = oracle.Basis(path, atoms).fourindex_eri(np.abs(p), 0.0)[:2]
+    for cut in (1.0, 1e30):
+        mixed = pa.Context(b, schwarz_tol=0.0, precision=pa.MIXED, mixed_cut=cut)
+        jm, km = mixed.fourindex_eri(p)
+        assert any(c["prec"] == "fp32" and c["kernel"] == "rys" and c["quartets"] for c in mixed.stats()["classes"])
+        f32 = 512 ** 0.5 * 2.0 ** -24
+        assert np.max(np.abs(jm - jr)) < f32 * np.max(np.abs(ja))
+        assert np.max(np.abs(km - kr)) < f32 * np.max(np.abs(ka))

@@ -1,7 +1,8 @@
 """Work buffers kept between calls: a call in blocks that an earlier call of
 other sizes left behind gives the result of a call in fresh ones (E(2) and
-CCSD of different molecules in turn, contexts alive and closed), and the last
-context's end gives the kept memory back."""
+CCSD of different molecules in turn, contexts alive and closed; gradients,
+periodic SCFs and k-point MP2 in turn), and the last context's end or a
+request gives the kept memory back."""
 import ctypes
 import gc
 
@@ -9,7 +10,7 @@ import numpy as np
 import pytest
 
 import polymer_amd as pa
-from polymer_amd import geometry
+from polymer_amd import geometry, run_polyethylene
 from polymer_amd._lib import check, lib
 from tests.molecules import BH_GOLDEN, H2O_GOLDEN
 
@@ -57,6 +58,46 @@ def test_reused_blocks_give_the_same_results():
         ctx.close()
     gc.collect()
     assert _free_bytes() > held
+
+
+def _gradient(n, basis):
+    b = pa.read_basis(basis, geometry.water_cluster(n, 1))
+    ctx = pa.Context(b)
+    rng = np.random.default_rng(n)
+    p = np.zeros((b.ncgs, b.ncgs))
+    a = 0.1 * rng.standard_normal((len(b.real_functions), 5 * n))
+    p[np.ix_(b.real_functions, b.real_functions)] = a @ a.T
+    return ctx, ctx.eri_gradient(p).ravel()
+
+
+def _polymer(units, kpoints):
+    period = 2.55 / pa.ANG_BOHR
+    atoms = [(z, x + u * period, y, w) for u in range(units) for z, x, y, w in run_polyethylene.cell()]
+    ctx = pa.Context(pa.read_basis("STO-3G", atoms), period=units * period, cel1=1, cel2=2)
+    r = ctx.self_consistent_field_periodic(kpoints=kpoints, scfconv=1e-9, diis=5, scfcycles=100)
+    e2 = ctx.mp2_energy_periodic(kpoints, r["co"], r["eps"], r["nall"], 2 * units, r["iocc"])
+    return ctx, np.array([r["e_total"], *e2])
+
+
+def test_blocks_pass_between_gradient_and_polymer_calls():
+    gc.collect()
+    jobs = [(_gradient, 1, "cc-pVDZ"), (_polymer, 1, 3), (_gradient, 3, "6-31Gss"), (_polymer, 2, 1), (_polymer, 1, 1)]
+    print("case: work buffers of gradient, periodic SCF and k-point MP2", flush=True)
+    fresh = []
+    for f, *args in jobs:
+        ctx, e = f(*args)
+        ctx.close()
+        fresh.append(e)
+    keep = []
+    for k in (3, 1, 0, 4, 2, 3, 0, 1, 2, 4):
+        f, *args = jobs[k]
+        ctx, e = f(*args)
+        keep.append(ctx)
+        assert np.max(np.abs(fresh[k])) > 1e-3
+        # the order of the atomics' sums: 10^5 terms of at most 10, 1.1e-10, first order in the orbitals' for E(2)
+        assert np.max(np.abs(e - fresh[k])) < (1.1e-10 if f is _gradient else 1e-8)
+    for ctx in keep:
+        ctx.close()
 
 
 def test_idle_blocks_are_given_back_on_request():
