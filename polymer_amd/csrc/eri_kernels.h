@@ -829,12 +829,11 @@ __device__ __forceinline__ double wave_sum(double v) {
 // lanes; without it every item has one lane.  BT: the block copies the
 // coarse Boys rows of its L into LDS, in front of the rows, and reads them
 // there.
-template <int LA, int LB, int LC, int LD, int MODE, bool SHARE, bool BT>
+template <int LA, int LB, int LC, int LD, bool SHARE, bool BT>
 __global__ void __launch_bounds__(256) k_eri_seg(EriArgs g) {
     constexpr int NA = ncart(LA), NB = ncart(LB), NC = ncart(LC), ND = ncart(LD);
     constexpr int NE = ((LA + LB + 1) * (LA + LB + 2) * (LA + LB + 3) - LA * (LA + 1) * (LA + 2)) / 6;
     constexpr int NF = ((LC + LD + 1) * (LC + LD + 2) * (LC + LD + 3) - LC * (LC + 1) * (LC + 2)) / 6;
-    using real = typename std::conditional<MODE == MODE_JK32, float, double>::type;
     extern __shared__ double lds_all[];
     const double* btab = g.boysA;
     double* seg_lds = lds_all;
@@ -891,15 +890,15 @@ __global__ void __launch_bounds__(256) k_eri_seg(EriArgs g) {
             const int nkp = !SHARE || live ? g.meta[kp].nprim : 0;
             const SoaKet kv{g.ksoa + g.bucket_soa[b] + (pos - g.bucket_start[b]),
                             g.bucket_start[b + 1] - g.bucket_start[b], g.kfs};
-            real acc[NE * NF];
+            double acc[NE * NF];
 #pragma unroll
-            for (int i = 0; i < NE * NF; ++i) acc[i] = real(0);
+            for (int i = 0; i < NE * NF; ++i) acc[i] = 0.0;
             // ket primitive outer (its fields stay in registers), bra inner
             // (the same for the whole block: scalar loads)
             for (int q = sub; q < nkp; q += 1 << ls) {
                 const PrimPair kq = kv.load(q);
                 for (int p = 0; p < mb.nprim; ++p)
-                    prim_vrr<real, LA, LB, LC, LD, BT>(scalar_load(bra + p), kq, btab, acc);
+                    prim_vrr<double, LA, LB, LC, LD, BT>(scalar_load(bra + p), kq, btab, acc);
             }
             if constexpr (SHARE) {
                 if (ls) {
@@ -910,11 +909,11 @@ __global__ void __launch_bounds__(256) k_eri_seg(EriArgs g) {
             }
             const PairMeta mk = g.meta[kp];
             const int fc = mk.fa, fd = mk.fb;
-            real v[NA * NB * NC * ND];
-            StoreCb<NB, NC, ND, real> st{v};
-            ClassCode<LA, LB, LC, LD, real>::hrr((real)ABx, (real)ABy, (real)ABz, (real)g.ab[4 * kp],
-                                                 (real)g.ab[4 * kp + 1], (real)g.ab[4 * kp + 2], acc, st);
-            RegDigest<NA, NB, NC, ND, real> cb;
+            double v[NA * NB * NC * ND];
+            StoreCb<NB, NC, ND, double> st{v};
+            ClassCode<LA, LB, LC, LD, double>::hrr(ABx, ABy, ABz, g.ab[4 * kp], g.ab[4 * kp + 1], g.ab[4 * kp + 2],
+                                                   acc, st);
+            RegDigest<NA, NB, NC, ND, double> cb;
             cb.load(g.D, n, fa, fb, fc, fd);
 #pragma unroll
             for (int a = 0; a < NA; ++a)
@@ -1417,10 +1416,10 @@ __global__ void __launch_bounds__(256) k_eri_gck(EriArgs g) {
 
 typedef void (*EriKernel)(EriArgs);
 // Getter modes of polyeri_class_kernel beyond the k_eri modes: the segment
-// kernel for MODE_JK and MODE_JK32, and for MODE_JK with items shared between
-// lanes; GET_SEG_SHARE_G is the last with the Boys rows read from global memory
-// (GET_SEG_JK and GET_SEG_SHARE need BOYS_CROWS doubles more LDS).
-enum { GET_SEG_JK = 5, GET_SEG_JK32 = 6, GET_SEG_SHARE = 7, GET_SEG_SHARE_G = 8 };
+// kernel (MODE_JK), the one with items shared between lanes, and the latter
+// with the Boys rows read from global memory (the first two need BOYS_CROWS
+// doubles more LDS).
+enum { GET_SEG_JK = 5, GET_SEG_SHARE = 6, GET_SEG_SHARE_G = 7 };
 // Strided batched FP64 products on the MFMA units (kgemm.hip):
 // C_b(m,n) = sum_k A_b(m,k) B_b(k,n), X_b(r,c) = X[b*sX + r*sXr + c*sXc].
 enum { GEMM_F64 = 1, GEMM_BF16X3 = 2 };
@@ -1540,8 +1539,8 @@ int polyeri_grad_launch(const GradArgs& g, double* d_grad, const hipStream_t* st
 // permuted together.  False (nothing changed) when a bound is not finite.
 bool polyeri_grad_sort_pairs(int* pa, int* pb, double* qp, int* pp0, int* pn, const int* seg);
 // The chunks of the pairs whose bound product is >= tol (sorted = false: of
-// all pairs, in their order); split: several lanes to a quartet.
-void polyeri_grad_chunks(const double* qp, const int* pn, const int* seg, double tol, bool sorted, bool split,
+// all pairs, in their order), with the lanes each quartet gets.
+void polyeri_grad_chunks(const double* qp, const int* pn, const int* seg, double tol, bool sorted,
                          GradChunks& ch);
 // the same sum on the host (host pointers), grad overwritten, Schwarz bounds
 // from gs

@@ -238,7 +238,7 @@ def main(out_path):
 
 def write_kernel_units(out_dir):
     """One translation unit per class (the five k_eri modes, and the segment
-    kernel as getter modes 5 and 6) plus the getter, so the class kernels
+    kernel's forms as getter modes 5 to 7) plus the getter, so the class kernels
     compile in parallel."""
     _, cls = classes()
     os.makedirs(out_dir, exist_ok=True)
@@ -256,8 +256,8 @@ def write_kernel_units(out_dir):
             body.append("    switch (mode) {")
             for m in range(5):
                 body.append(f"    case {m}: return k_eri<{la}, {lb}, {lc}, {ld}, {m}>;")
-            # getter modes 5 .. 8: the forms of the segment kernel
-            for m, form in ((5, "0, false, true"), (6, "3, false, false"), (7, "0, true, true"), (8, "0, true, false")):
+            # getter modes 5 .. 7: the forms of the segment kernel
+            for m, form in ((5, "false, true"), (6, "true, true"), (7, "true, false")):
                 body.append(f"    case {m}: return k_eri_seg<{la}, {lb}, {lc}, {ld}, {form}>;")
             body += ["    }", "    return nullptr;", "}", ""]
         text = "\n".join(body)

@@ -8,10 +8,9 @@ EriKernel polyeri_kernel_2011(int mode) {
     case 2: return k_eri<2, 0, 1, 1, 2>;
     case 3: return k_eri<2, 0, 1, 1, 3>;
     case 4: return k_eri<2, 0, 1, 1, 4>;
-    case 5: return k_eri_seg<2, 0, 1, 1, 0, false, true>;
-    case 6: return k_eri_seg<2, 0, 1, 1, 3, false, false>;
-    case 7: return k_eri_seg<2, 0, 1, 1, 0, true, true>;
-    case 8: return k_eri_seg<2, 0, 1, 1, 0, true, false>;
+    case 5: return k_eri_seg<2, 0, 1, 1, false, true>;
+    case 6: return k_eri_seg<2, 0, 1, 1, true, true>;
+    case 7: return k_eri_seg<2, 0, 1, 1, true, false>;
     }
     return nullptr;
 }

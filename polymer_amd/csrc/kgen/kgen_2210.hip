@@ -8,10 +8,9 @@ EriKernel polyeri_kernel_2210(int mode) {
     case 2: return k_eri<2, 2, 1, 0, 2>;
     case 3: return k_eri<2, 2, 1, 0, 3>;
     case 4: return k_eri<2, 2, 1, 0, 4>;
-    case 5: return k_eri_seg<2, 2, 1, 0, 0, false, true>;
-    case 6: return k_eri_seg<2, 2, 1, 0, 3, false, false>;
-    case 7: return k_eri_seg<2, 2, 1, 0, 0, true, true>;
-    case 8: return k_eri_seg<2, 2, 1, 0, 0, true, false>;
+    case 5: return k_eri_seg<2, 2, 1, 0, false, true>;
+    case 6: return k_eri_seg<2, 2, 1, 0, true, true>;
+    case 7: return k_eri_seg<2, 2, 1, 0, true, false>;
     }
     return nullptr;
 }

@@ -71,7 +71,7 @@ bool polyeri_grad_sort_pairs(int* pa, int* pb, double* qp, int* pp0, int* pn, co
     return true;
 }
 
-void polyeri_grad_chunks(const double* qp, const int* pn, const int* seg, double tol, bool sorted, bool split,
+void polyeri_grad_chunks(const double* qp, const int* pn, const int* seg, double tol, bool sorted,
                          GradChunks& ch) {
     ch.off.clear();
     ch.ij.clear();
@@ -124,7 +124,7 @@ void polyeri_grad_chunks(const double* qp, const int* pn, const int* seg, double
             unsigned long long tot = 0;
             for (int c = 0; c < ch.n[k]; ++c) {
                 int& u = ch.ij[ch.ij0[k] + 3 * c + 2];
-                u = split ? (int)std::min<double>(std::max(1.0, std::ceil(u / grain)), kGradMaxLanes) : 1;
+                u = (int)std::min<double>(std::max(1.0, std::ceil(u / grain)), kGradMaxLanes);
                 ch.off.push_back(tot);
                 tot += (unsigned long long)ni[c] * u;
             }
@@ -170,7 +170,7 @@ int polyeri_grad_host(const GradArgs& g, const GradShells& gs, double* grad) {
         pn(g.pn, g.pn + npair);
     const bool sorted = polyeri_grad_sort_pairs(pa.data(), pb.data(), Qp.data(), pp0.data(), pn.data(), g.seg);
     GradChunks ch;
-    polyeri_grad_chunks(Qp.data(), pn.data(), g.seg, g.tol, sorted, true, ch);
+    polyeri_grad_chunks(Qp.data(), pn.data(), g.seg, g.tol, sorted, ch);
     GradArgs gq = g;
     gq.Qp = Qp.data();
     gq.pa = pa.data();

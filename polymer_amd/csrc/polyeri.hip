@@ -765,7 +765,7 @@ static int launch_class(polyeri_ctx* c, int mode, int la, int lb, int lc, int ld
     if (kind == LAUNCH_SEG && !seg_ok) kind = k ? LAUNCH_REG : LAUNCH_COOP;
     if (kind == LAUNCH_REG && !k) return fail(POLYERI_E_ARG, "no register kernel for class");
     if (kind == LAUNCH_SEG && mode == MODE_JK32)
-        return fail(POLYERI_E_ARG, "the FP32 segment kernel is switched off (unexplained fault)");
+        return fail(POLYERI_E_ARG, "the light classes have no FP32 segment kernel");
     if (kind == LAUNCH_RYS) {
         const bool rys_ok = seg_ok && polyeri_rys_class(la, lb, lc, ld) &&
                             polyeri_rys_lds_bytes(la, lb, c->ib.nbf) <= 65536;
@@ -786,13 +786,9 @@ static int launch_class(polyeri_ctx* c, int mode, int la, int lb, int lc, int ld
     if (kind == LAUNCH_SEG) {
         // the coarse Boys rows go into LDS where they fit beside the rows
         size_t lds = seg_lds_bytes(la, lb, c->ib.nbf);
-        const bool bt = mode == MODE_JK && lds + BOYS_CROWS * sizeof(double) <= 65536;
+        const bool bt = lds + BOYS_CROWS * sizeof(double) <= 65536;
         if (bt) lds += BOYS_CROWS * sizeof(double);
-        EriKernel ks = polyeri_class_kernel(la, lb, lc, ld,
-                                            mode != MODE_JK ? GET_SEG_JK32
-                                            : !bt           ? GET_SEG_SHARE_G
-                                            : share         ? GET_SEG_SHARE
-                                                            : GET_SEG_JK);
+        EriKernel ks = polyeri_class_kernel(la, lb, lc, ld, !bt ? GET_SEG_SHARE_G : share ? GET_SEG_SHARE : GET_SEG_JK);
         if (!ks) return fail(POLYERI_E_ARG, "no segment kernel for class");
         a.segs = segs;
         a.nseg = nseg;
@@ -1296,8 +1292,8 @@ static int build_ctx(polyeri_ctx* c) {
     // splits the class pairs of the wavefront kernel only: the light classes
     // keep one FP64 list each and run the segment and generally contracted
     // kernels, as in FP64 contexts (an FP32 recursion issues at the FP64 rate
-    // on gfx950 without packed FP32 math, so it saves them nothing, and the
-    // FP32 segment kernel stays switched off; see launch_class).
+    // on gfx950 without packed FP32 math, so it saves them nothing, and there
+    // is no FP32 segment kernel for them; see the segment lists below).
     std::vector<WorkList> wl;
     const double cut = c->opts.precision == POLYERI_MIXED ? c->opts.mixed_cut : 0.0;
     uint64_t split = 0;
@@ -1377,12 +1373,12 @@ static int build_ctx(polyeri_ctx* c) {
         HIPCHK(hipMemcpy(w.d_row, l.row.data(), l.row.size() * sizeof(long long), hipMemcpyHostToDevice));
         if (!l.rb.empty()) HIPCHK(hipMemcpy(w.d_rb, l.rb.data(), l.rb.size() * sizeof(int), hipMemcpyHostToDevice));
         // Segment lists for the FP64 lists of molecular contexts, and for the
-        // FP32 lists of the Rys classes (their own kernel).  The light FP32
-        // lists get none: the FP32 light-class segment kernel once stopped on
-        // an illegal memory access ((H2O)4 cc-pVDZ, cut 1e-5) whose cause is
-        // not established (a host replay of its index path over those lists
-        // stays in bounds), so it is not launched, and mixed contexts do not
-        // split the light classes.
+        // FP32 lists of the Rys classes (their own kernel).  Light FP32 lists
+        // do not exist (mixed contexts do not split the light classes) and
+        // would get none: an FP32 form of the light-class segment kernel once
+        // stopped on an illegal memory access ((H2O)4 cc-pVDZ, cut 1e-5) whose
+        // cause was not established (a host replay of its index path over
+        // those lists stayed in bounds), so that form is not built.
         if (!c->pbc && l.nwork > 0 && (!l.prec || polyeri_rys_class(w.la, w.lb, w.lc, w.ld))) {
             const bool rys = polyeri_rys_class(w.la, w.lb, w.lc, w.ld);
             sl.build(l, c->pairs, c->class_ids[l.X], c->ket_ids[l.Y], c->bstart[l.Y], kq[l.Y], all, rys);
@@ -4430,7 +4426,7 @@ int polyeri_eri_gradient(polyeri_ctx* ctx, const double* p_c, double hfexchange,
     if ((rc = grad_pair_prims(ctx->pairs, &ctx->Q, h, &qp))) return rc;
     const bool sorted = polyeri_grad_sort_pairs(h.pa.data(), h.pb.data(), qp.data(), h.pp0.data(), h.pn.data(), h.seg);
     GradChunks ch;
-    polyeri_grad_chunks(qp.data(), h.pn.data(), h.seg, ctx->opts.schwarz_tol, sorted, true, ch);
+    polyeri_grad_chunks(qp.data(), h.pn.data(), h.seg, ctx->opts.schwarz_tol, sorted, ch);
     DevBuf buf(ctx->stream);
     int *dAt, *dF0, *dPa, *dPb, *dPp, *dPn, *dIj;
     double *dXyz, *dD, *dDsh, *dQp, *dG;
