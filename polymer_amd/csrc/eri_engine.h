@@ -35,9 +35,11 @@
 #define BOYS_AOFF (BOYS_NT * BOYS_NM)
 // A third layout, small enough for LDS, for the kernels that copy it there:
 // for each L < BOYS_LC, rows of ten coefficients F_{l+k}(T_j) / k! on the
-// coarse grid T_j = 3 j / 20 (every third point of the main grid; the last
-// row also serves T up to BOYS_TMAX).  |h| <= 0.075 leaves less than 3e-17 of
-// the result.  It follows the aligned tables (BOYS_COFF doubles in);
+// coarse grid T_j = 3 j / 20 (every third point of the main grid).  F_L is the
+// derivative of the polynomial, nine terms: |h| <= 0.075 leaves h^9 / 9! x
+// F_{L+9}(T) / F_L(T) of it, from 3e-17 (L = 1) to 9e-17 (L = 6) at T = 0 and less beyond.
+// The last row also serves T up to BOYS_TMAX, |h| <= 0.1, where F_{L+9} / F_L
+// is below 5e-6.  It follows the aligned tables (BOYS_COFF doubles in);
 // BOYS_CROWS doubles (21 360 bytes) per L.
 #define BOYS_LC 7
 #define BOYS_CNT 267

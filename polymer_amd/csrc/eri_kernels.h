@@ -814,8 +814,8 @@ __device__ __forceinline__ void lane_reduce(double* acc, int ls, int lane, int& 
 // registers (J_ab, reduced over the wavefront), and added to the XCD's J/K
 // copy once per segment, one atomic per nonzero element.  Only J_cd is added
 // per quartet.  LDS: ((NA + NB) nbf + NA NB) doubles.
-// Bound by the loads and atomics of the digestion (texture data path 60-75 %
-// busy, FP64 VALU 25-60 %).  With the ket primitive outside, the bra's in
+// Bound by the loads and atomics of the digestion (texture data path 29-66 %
+// busy, FP64 VALU 16-46 %, over the classes of (H2O)16 cc-pVDZ).  With the ket primitive outside, the bra's in
 // scalar registers and the Boys rows in LDS no vector load is left in the
 // inner loop: C16H34 6-31G** (ss|ss) 0.69 -> 0.44, (ps|ss) 1.18 -> 0.89 ms,
 // (H2O)16 cc-pVDZ (pp|ss) 1.38 -> 0.95, (pp|ps) 1.63 -> 1.49 ms.
@@ -968,18 +968,19 @@ __global__ void __launch_bounds__(256) k_eri_seg(EriArgs g) {
     }
 }
 
-// Segment kernel of the generally contracted lists, classes (ls|l's)
-// ((H2O)16: (ss|ss) 2.9 -> 1.2 ms with shared items and scalar bra loads,
-// (ps|ss) 3.1 -> 2.2, (ps|ps) 2.6 -> 1.9; FP64 VALU 38-53 % busy): as
+// Segment kernel of the generally contracted lists, classes (ls|l's): as
 // k_eri_seg, but an item is a pair of generally contracted pairs (GcMeta)
 // and computes all member quartets from one primitive loop: for each ket
 // primitive, the primitive quartets' [a0|c0] blocks are summed over the bra
 // primitives with each bra member's weights, and that sum is added to every
 // member quartet with the ket members' weights.  Each member quartet
-// that passes the Schwarz test is digested with its own degeneracy weight; a list row whose bra equals
-// the ket visits both orders of two different members, each at half
-// weight.  LDS: the exchange rows of the up to two shells of each bra group
-// ((2 NA + 2) nbf doubles) and J_ab of every bra member (MB NA doubles).
+// that passes the Schwarz test is digested with its own degeneracy weight; a
+// list row whose bra equals the ket visits both orders of two different
+// members, each at half weight.  LDS: the exchange rows of the up to two
+// shells of each bra group ((2 NA + 2) nbf doubles) and J_ab of every bra
+// member (MB NA doubles).  (H2O)16 cc-pVDZ: (ss|ss) 2.9 -> 1.2 ms with shared
+// items and scalar bra loads, (ps|ss) 3.1 -> 2.2, (ps|ps) 2.6 -> 1.9; texture
+// data path 41-77 % busy, FP64 VALU 33-51 %.
 // Largest shell-block density maximum between shells {x0, x1} and {y0, y1}
 // (x1 / y1 < 0: absent).
 __device__ __forceinline__ double gc_dmax(const EriArgs& g, int x0, int x1, int y0, int y1) {

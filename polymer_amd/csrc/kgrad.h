@@ -331,6 +331,9 @@ POLY_HD void grad_units(const GradArgs& g, const RysTabs& rt, int pij, int pkl, 
         const double PA[3] = {bq.PAx, bq.PAy, bq.PAz}, QC[3] = {kq.PAx, kq.PAy, kq.PAz};
         const double T = bq.zeta * roz * (PQ[0] * PQ[0] + PQ[1] * PQ[1] + PQ[2] * PQ[2]);
         const double pref = fdeg * bq.K * kq.K * rs;
+        // 2 beta by difference: it rounds by 2^-53 zeta / beta of it, where the
+        // pair's prefactor has fallen as fast (against the exponents themselves
+        // 1e-14 of the largest component in cc-pVDZ, 1.5e-13 at zeta / beta = 1e8)
         const double be2 = 2.0 * bq.zeta - bq.a2;
         const int r0 = ROOTS ? w - pq * NR : 0, r1 = ROOTS ? r0 + 1 : NR;
 #pragma unroll
